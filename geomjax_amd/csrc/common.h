@@ -21,19 +21,22 @@ namespace gjx {
 //   row_half_mirror = 0x141 (lane i <-> 7-i in each half row),
 //   row_mirror = 0x140 (lane i <-> 15-i in each row).
 // After the two quad steps all lanes of a quad hold the quad total, so the
-// mirror steps pair whole quads / half rows, as an xor butterfly would.
+// mirror steps pair whole quads / half rows, as an xor butterfly would.  Every
+// control used here reads a valid lane, so bound_ctrl (zero for lanes without a
+// source) never acts; with it set the move needs no initialised destination and
+// the compiler folds it into the float32 add or max that follows.
 // ---------------------------------------------------------------------------
 template <int CTRL>
 __device__ __forceinline__ float dpp_f32(float v) {
   return __builtin_bit_cast(
-      float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), CTRL, 0xF, 0xF, false));
+      float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), CTRL, 0xF, 0xF, true));
 }
 
 template <int CTRL>
 __device__ __forceinline__ double dpp_f64(double v) {
   uint64_t b = __builtin_bit_cast(uint64_t, v);
-  int lo = __builtin_amdgcn_update_dpp(0, (int)(uint32_t)b, CTRL, 0xF, 0xF, false);
-  int hi = __builtin_amdgcn_update_dpp(0, (int)(uint32_t)(b >> 32), CTRL, 0xF, 0xF, false);
+  int lo = __builtin_amdgcn_update_dpp(0, (int)(uint32_t)b, CTRL, 0xF, 0xF, true);
+  int hi = __builtin_amdgcn_update_dpp(0, (int)(uint32_t)(b >> 32), CTRL, 0xF, 0xF, true);
   return __builtin_bit_cast(double, ((uint64_t)(uint32_t)hi << 32) | (uint32_t)lo);
 }
 

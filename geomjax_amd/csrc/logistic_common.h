@@ -1,17 +1,28 @@
 // Device routines of the float64 logistic-regression kernels (Fisher metric):
-// LDS layout, chunked passes over X with MFMA Gram / quadratic forms, the
-// symmetric sweep inverse and the Cholesky used for momentum draws.
+// LDS layout, passes over X with MFMA Gram / quadratic forms, the symmetric
+// sweep inverse and the Cholesky used for momentum draws.
 //
 // One workgroup of NT = 256 lanes (4 waves) per chain.  Everything is
 // parameterised by the feature capacity MD (64 or 128) through Cfg<MD>:
-//   RCH  rows of X per LDS chunk (32, or 16 so that a 128 x 128 float64
-//        inverse and the chunk fit the 160 KiB of LDS together),
-//   LDX  padded row stride, TB 16-wide tiles per dimension, NLT lower tiles of
-//        the Gram, TPW tiles per wave, BS the BS x BS block of the inverse each
-//        lane holds during the sweep (16 x 16 lanes cover the matrix),
-//   TPR  lanes per row in the per-row passes (CPT = 8 columns each), RG row
-//        groups of the column-per-lane accumulations (X^T r, X^T h, G v).
+//   TB 16-wide tiles per dimension, NLT lower tiles of the Gram, BS the BS x BS
+//   block of the inverse each lane holds during the sweep (16 x 16 lanes cover
+//   the matrix), LDX the padded LDS row stride of the matrix.
+//
+// Passes over X.  Each wave takes whole 16-row blocks (block w, w + 4, ...) and
+// reads them from global memory (L2: all chains of a posterior share X) straight
+// into the operand layout of v_mfma_f64_16x16x4f64, so the loops hold no barrier
+// and no LDS staging; the waves' partial sums meet in LDS once per pass.  Bound:
+// the float64 matrix pipe, 64 cycles an MFMA and 40 MFMAs per 16 rows and pass at
+// D = 64 (40 us a pass and workgroup at 2.07 GHz), plus the passes' own VALU
+// instructions, which do not overlap float64 MFMAs (measured: 4 cycles added
+// per instruction, float32 ones too).  At 2048 x 64 with two workgroups on a CU a
+// Gram pass takes 50 us, a quadratic-form pass 51, a sweep 12 per workgroup.  The
+// form before (32-row chunks of X staged in LDS behind four barriers each, the
+// tiles dealt to the waves 3, 3, 2, 2, 64 MFMAs per 16 rows in the second
+// pass) made a transition of 1024 chains, 10 steps, 107.5 ms; this one 30.7 ms.
 #pragma once
+
+#include <type_traits>
 
 #include "common.h"
 
@@ -24,53 +35,31 @@ template <int MD>
 struct Cfg {
   static_assert(MD == 64 || MD == 128, "feature capacity 64 or 128");
   static constexpr int MAXD = MD;
-  static constexpr int RCH = MD == 64 ? 32 : 16;
   static constexpr int LDX = MD + 1;
   static constexpr int TB = MD / 16;
   static constexpr int NLT = TB * (TB + 1) / 2;
-  static constexpr int TPW = (NLT + 3) / 4;
   static constexpr int BS = MD / 16;
-  static constexpr int TPR = NT / RCH;
-  static constexpr int CPT = MD / TPR;
-  static constexpr int RG = NT / MD;
-  static constexpr int CB2 = TB / 2;          // column-block pairs of the quadratic-form pass
-  static constexpr int RB = RCH / 16;         // 16-row blocks per chunk
-  static_assert(RB * CB2 == 4, "the quadratic-form pass gives each wave one (row block, column pair)");
+  // Gram pass: the waves form H groups, each with its share of the tiles (288
+  // registers of tiles at 128 features do not leave room for the rows)
+  static constexpr int H = MD == 64 ? 1 : 2;
 };
 
 typedef double f64x4 __attribute__((ext_vector_type(4)));
 
 template <class C>
 struct Smem {
-  // the chunk of X; outside the chunk loops its space holds the sweep's row
-  // broadcast and the partial sums of the column-per-lane accumulations
   union {
-    double Xs[C::RCH * C::LDX];
-    struct {
-      double rowbuf[2][C::MAXD];
-      double part[4][C::MAXD];
-    };
+    double Gi[C::MAXD * C::LDX];        // G, then the Cholesky factor or G^-1
+    double tile[2 * (C::NLT / C::H) * 256];  // two waves' partial Gram tiles at the end of a Gram pass
   };
-  double Gi[C::MAXD * C::LDX];  // G, then the Cholesky factor or G^-1
-  double yv[C::RCH];
-  double lam[C::RCH];  // lambda (pass 1) / w (pass 2)
-  double rr[C::RCH];   // y - s
-  double bb[C::RCH];   // x_n . u
-  double aa[4][C::RCH];
-  double hh[C::RCH];
+  double rowbuf[2][C::MAXD];  // sweep: the pivot row
+  double part[4][C::MAXD];    // the waves' partial sums of X^T r, X^T h, G v
+  double dk[C::MAXD];         // pivots of the last sweep
   double q0[C::MAXD], p0[C::MAXD], q[C::MAXD], p[C::MAXD], u[C::MAXD], dH[C::MAXD], g[C::MAXD], z[C::MAXD],
       qs[C::MAXD];
   double gv[C::MAXD], vt[C::MAXD];
   double red[8];
 };
-
-// the lower-triangular 16 x 16 tiles (bi >= bj) in the order (0,0),(1,0),(1,1),(2,0),...
-__device__ __forceinline__ void tile_of(int t, int& bi, int& bj) {
-  int i = 0;
-  while ((i + 1) * (i + 2) / 2 <= t) ++i;
-  bi = i;
-  bj = t - i * (i + 1) / 2;
-}
 
 template <class C>
 __device__ __forceinline__ double block_sum(Smem<C>& S, double v) {
@@ -95,128 +84,316 @@ __device__ __forceinline__ double block_max(Smem<C>& S, double v) {
 __device__ __forceinline__ double softplus(double x) { return fmax(x, 0.0) + log1p(exp(-fabs(x))); }
 __device__ __forceinline__ double sigmoid(double x) { return 1.0 / (1.0 + exp(-x)); }
 
-// Stage rows [n0, n0 + RCH) of X (zero-padded past N and D) and y into LDS.
-template <class C>
-__device__ __forceinline__ void load_chunk(Smem<C>& S, const double* X, const double* y, int N, int D, int n0) {
-  const int t = threadIdx.x;
-  const int r = t / (C::MAXD / 8), c0 = (t % (C::MAXD / 8)) * 8;
-  const int n = n0 + r;
-#pragma unroll
-  for (int e = 0; e < 8; ++e) {
-    const int col = c0 + e;
-    S.Xs[r * C::LDX + col] = (n < N && col < D) ? X[(size_t)n * D + col] : 0.0;
-  }
-  if (t < C::RCH) S.yv[t] = (n0 + t < N) ? y[n0 + t] : 0.0;
+// Sum over the four 16-lane rows of the wave (lanes l, l ^ 16, l ^ 32, l ^ 48),
+// the same in all four.
+__device__ __forceinline__ double rows_sum(double v) {
+  const uint64_t b = __builtin_bit_cast(uint64_t, v);
+  const auto lo = __builtin_amdgcn_permlane16_swap((uint32_t)b, (uint32_t)b, false, false);
+  const auto hi = __builtin_amdgcn_permlane16_swap((uint32_t)(b >> 32), (uint32_t)(b >> 32), false, false);
+  const double s = __builtin_bit_cast(double, ((uint64_t)hi[0] << 32) | lo[0]) +
+                   __builtin_bit_cast(double, ((uint64_t)hi[1] << 32) | lo[1]);
+  const uint64_t c = __builtin_bit_cast(uint64_t, s);
+  const auto lo2 = __builtin_amdgcn_permlane32_swap((uint32_t)c, (uint32_t)c, false, false);
+  const auto hi2 = __builtin_amdgcn_permlane32_swap((uint32_t)(c >> 32), (uint32_t)(c >> 32), false, false);
+  return __builtin_bit_cast(double, ((uint64_t)hi2[0] << 32) | lo2[0]) +
+         __builtin_bit_cast(double, ((uint64_t)hi2[1] << 32) | lo2[1]);
 }
 
-// Sum of the RG row-group partials of a column-per-lane accumulation: lane
-// t < MAXD receives column t's total.
-template <class C>
-__device__ __forceinline__ double column_total(Smem<C>& S, int t) {
-  double s = 0.0;
-#pragma unroll
-  for (int g = 0; g < C::RG; ++g) s += S.part[g][t];
-  return s;
+// Sums of four values over the 16 lanes of a row, one per lane: lane l receives
+// the total of e[l % 4] (the four lanes with that l % 4 the same bits).
+__device__ __forceinline__ double sum4_of_16(const double (&e)[4], int l) {
+  const bool b0 = l & 1, b1 = l & 2;
+  const double k0 = (b0 ? e[1] : e[0]) + dpp<0xB1>(b0 ? e[0] : e[1]);
+  const double k1 = (b0 ? e[3] : e[2]) + dpp<0xB1>(b0 ? e[2] : e[3]);
+  double v = (b1 ? k1 : k0) + dpp<0x4E>(b1 ? k0 : k1);
+  v += dpp<0x128>(v);         // row_ror 8
+  return v + dpp<0x124>(v);  // row_ror 4
+}
+
+// v of lane J of each quad
+template <int J>
+__device__ __forceinline__ double quad_bcast(double v) { return dpp<J * 0x55>(v); }
+
+// f(integral_constant<NB>) for the number of 16-feature tiles of a posterior
+// with D features (capacity 128: six or eight tiles).
+template <class C, class F>
+__device__ __forceinline__ void by_width(int D, F f) {
+  if constexpr (C::MAXD == 64) {
+    if (D <= 16) f(std::integral_constant<int, 1>{});
+    else if (D <= 32) f(std::integral_constant<int, 2>{});
+    else if (D <= 48) f(std::integral_constant<int, 3>{});
+    else f(std::integral_constant<int, 4>{});
+  } else {
+    if (D <= 96) f(std::integral_constant<int, 6>{});
+    else f(std::integral_constant<int, 8>{});
+  }
 }
 
 // Gram pass at S.q: S.Gi = X^T diag(lambda + coef w (X vec)) X + I / prior_var
-// (vec == nullptr: the Fisher metric G itself).  With want_lg it also returns
-// the log-likelihood sum and leaves grad l = X^T (y - s) - q/prior_var in S.g;
-// with want_gv it leaves G vec = X^T (lambda (X vec)) + vec/prior_var in S.gv.
-template <class C>
-__device__ void pass_gram(Smem<C>& S, const double* X, const double* y, int N, int D, double prior_var,
-                          const double* vec, double coef, bool want_lg, bool want_gv, double& loglik) {
-  const int t = threadIdx.x, w = t / 64, l = t % 64;
-  const int nb = (D + 15) / 16;
-  f64x4 acc[C::TPW];
+// (vec == nullptr: the Fisher metric G itself) in the first D rows and columns
+// (nothing meaningful past them: load_block reads zeros there).  With want_lg it
+// also returns the log-likelihood sum and leaves grad l = X^T (y - s) - q/prior_var
+// in S.g; with want_gv it leaves G vec = X^T (lambda (X vec)) + vec/prior_var in
+// S.gv.  S.q and vec are zero past D over the capacity.
+//
+// NB = ceil(D / 16) feature tiles.  Lane l = 16 g + m holds X[n0 + 4 j + g][16 b + m]
+// (j < 4, b < NB) of a 16-row block: for each j both operands of the K step of rows
+// 4 j .. 4 j + 3.  eta of the lane's row n0 + 4 (l % 4) + g comes from a reduce-scatter
+// over the 16 lanes, so the sigmoid is evaluated once per row and four lanes; the
+// weight of K step j is lane j's of each quad.
+// Tiles T0 .. T0 + NT of the lower triangle, for the wave's share of the rows: blocks
+// w, w + WR, ...
+template <class C, int NB, int T0, int NTW, bool VEC, bool LG>
+__device__ __forceinline__ void gram_loop(Smem<C>& S, const double* X, const double* y, int N, int D, const double* vec,
+                                          double coef, bool want_gv, int w, f64x4 (&acc)[NTW], double& ll,
+                                          double (&gacc)[NB], double (&gvacc)[NB]) {
+  constexpr int WR = 4 / C::H;
+  const int l = threadIdx.x % 64;
+  const int g = l / 16, m = l % 16;
+  const int nblk = (N + 15) / 16;
+  if (nblk == 0) return;
+  double qv[NB], vv[VEC ? NB : 1];
 #pragma unroll
-  for (int m = 0; m < C::TPW; ++m) acc[m] = f64x4{0, 0, 0, 0};
-  double ll = 0.0, gacc = 0.0, gvacc = 0.0;
-  for (int n0 = 0; n0 < N; n0 += C::RCH) {
-    load_chunk(S, X, y, N, D, n0);
-    __syncthreads();
-    {
-      const int r = t / C::TPR, c0 = (t % C::TPR) * C::CPT;
-      double eta = 0.0, xv = 0.0;
-#pragma unroll
-      for (int e = 0; e < C::CPT; ++e) {
-        eta += S.Xs[r * C::LDX + c0 + e] * S.q[c0 + e];
-        if (vec) xv += S.Xs[r * C::LDX + c0 + e] * vec[c0 + e];
-      }
-      eta = group_sum<C::TPR>(eta);
-      if (vec) xv = group_sum<C::TPR>(xv);
-      if (t % C::TPR == 0) {
-        const bool ok = n0 + r < N;
-        const double s = sigmoid(eta);
-        const double lam = s * (1.0 - s);
-        S.lam[r] = ok ? (vec ? lam + coef * lam * (1.0 - 2.0 * s) * xv : lam) : 0.0;
-        S.rr[r] = ok ? S.yv[r] - s : 0.0;
-        S.bb[r] = ok ? lam * xv : 0.0;
-        if (want_lg && ok) ll += S.yv[r] * eta - softplus(eta);
-      }
-    }
-    __syncthreads();
-    // Gram tiles on MFMA: K steps of 4 rows
-#pragma unroll 2
-    for (int ks = 0; ks < C::RCH / 4; ++ks) {
-      const int nr = ks * 4 + l / 16;
-      double xb[C::TB];
-#pragma unroll
-      for (int b = 0; b < C::TB; ++b) xb[b] = S.Xs[nr * C::LDX + b * 16 + l % 16];
-      const double lm = S.lam[nr];
-#pragma unroll
-      for (int m = 0; m < C::TPW; ++m) {
-        const int tt = w + 4 * m;
-        if (tt >= C::NLT) continue;
-        int bi, bj;
-        tile_of(tt, bi, bj);
-        if (bi >= nb) continue;
-        acc[m] = __builtin_amdgcn_mfma_f64_16x16x4f64(lm * xb[bi], xb[bj], acc[m], 0, 0, 0);
-      }
-    }
-    if (want_lg || want_gv) {
-      const int k = t % C::MAXD;
-#pragma unroll
-      for (int m = 0; m < C::RCH / C::RG; ++m) {
-        const int r = t / C::MAXD + C::RG * m;
-        const double xk = S.Xs[r * C::LDX + k];
-        gacc += xk * S.rr[r];
-        gvacc += xk * S.bb[r];
-      }
-    }
-    __syncthreads();
+  for (int b = 0; b < NB; ++b) {
+    qv[b] = S.q[16 * b + m];
+    if constexpr (VEC) vv[b] = vec[16 * b + m];
   }
-  // tiles -> S.Gi (both triangles), C[4r + l/16][l%16] layout
+  struct Blk {
+    double x[4][NB];
+    double y;
+  };
+  // features past D in the last tile read feature D - 1, rows past N row N - 1
+  // (in bounds; they meet zeros or tile entries that are not used); past its
+  // last block a wave re-reads the last one with weights of zero
+  // (byte offsets from a block's first row: a uniform base, one 32-bit lane offset
+  // per K step and immediate offsets per tile)
+  const uint32_t mb = 8u * (uint32_t)m, lastb = 8u * (uint32_t)min(16 * (NB - 1) + m, D - 1);
+  uint32_t rowb[4];
 #pragma unroll
-  for (int m = 0; m < C::TPW; ++m) {
-    const int tt = w + 4 * m;
-    if (tt >= C::NLT) continue;
-    int bi, bj;
-    tile_of(tt, bi, bj);
+  for (int j = 0; j < 4; ++j) rowb[j] = 8u * (uint32_t)((4 * j + g) * D);
+  auto fetch_row = [&](Blk& B, int blk, int j) {
+    const int n0 = 16 * min(blk, nblk - 1);
+    const char* const Xb = reinterpret_cast<const char*>(X + (size_t)n0 * D);
+    const uint32_t row = min(rowb[j], 8u * (uint32_t)(min(N - n0 - 1, 15) * D));
+    const double* const xr = reinterpret_cast<const double*>(Xb + (row + mb));
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int i = bi * 16 + 4 * r + l / 16, j = bj * 16 + l % 16;
-      // a diagonal tile holds (i, j) and (j, i) rounded differently: keep the
-      // lower one for both so that G is exactly symmetric
-      if (i < j) continue;
-      double v = acc[m][r];
-      if (i == j && i < D) v += 1.0 / prior_var;
-      S.Gi[i * C::LDX + j] = v;
-      S.Gi[j * C::LDX + i] = v;
+    for (int b = 0; b < NB - 1; ++b) B.x[j][b] = xr[16 * b];
+    B.x[j][NB - 1] = *reinterpret_cast<const double*>(Xb + (row + lastb));
+  };
+  auto fetch_y = [&](Blk& B, int blk) {
+    const int n0 = 16 * min(blk, nblk - 1);
+    if constexpr (LG) B.y = (y + n0)[min(4 * (l & 3) + g, N - n0 - 1)];
+  };
+  struct Wt {
+    double lam, rr, bb;
+  };
+  auto weights = [&](const Blk& B, int blk, Wt& o) {
+    double e[4], v[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      e[j] = 0.0;
+      v[j] = 0.0;
+#pragma unroll
+      for (int b = 0; b < NB; ++b) {
+        e[j] = fma(B.x[j][b], qv[b], e[j]);
+        if constexpr (VEC) v[j] = fma(B.x[j][b], vv[b], v[j]);
+      }
+    }
+    const double eta = sum4_of_16(e, l);
+    const bool ok = 16 * blk + 4 * (l & 3) + g < N;
+    const double s = sigmoid(eta);
+    const double lam = s * (1.0 - s);
+    o.lam = ok ? lam : 0.0;
+    if constexpr (VEC) {
+      const double xv = sum4_of_16(v, l);
+      o.lam = ok ? lam + coef * lam * (1.0 - 2.0 * s) * xv : 0.0;
+      o.bb = ok ? lam * xv : 0.0;
+    }
+    if constexpr (LG) {
+      o.rr = ok ? B.y - s : 0.0;
+      if (ok && m < 4) ll += B.y * eta - softplus(eta);
+    }
+  };
+  auto kstep = [&](const Blk& B, const Wt& o, auto jc) {
+    constexpr int j = decltype(jc)::value;
+    const double lm = quad_bcast<j>(o.lam);
+    double xl[NB];
+#pragma unroll
+    for (int b = 0; b < NB; ++b) xl[b] = lm * B.x[j][b];
+    int t = 0;
+#pragma unroll
+    for (int bi = 0; bi < NB; ++bi)
+#pragma unroll
+      for (int bj = 0; bj <= bi; ++bj) {
+        if (t >= T0 && t < T0 + NTW)
+          acc[t - T0] = __builtin_amdgcn_mfma_f64_16x16x4f64(xl[bi], B.x[j][bj], acc[t - T0], 0, 0, 0);
+        ++t;
+      }
+    if constexpr (LG) {
+      const double r = quad_bcast<j>(o.rr);
+#pragma unroll
+      for (int b = 0; b < NB; ++b) gacc[b] = fma(B.x[j][b], r, gacc[b]);
+    }
+    if constexpr (VEC) {
+      if (want_gv) {
+        const double r = quad_bcast<j>(o.bb);
+#pragma unroll
+        for (int b = 0; b < NB; ++b) gvacc[b] = fma(B.x[j][b], r, gvacc[b]);
+      }
+    }
+  };
+  // One register set: each K step's rows are reloaded for the next block as soon
+  // as its MFMAs are issued (the scheduling barriers keep the loads there: hoisted,
+  // they need a second set and spill); the second wave of the SIMD covers the
+  // latency of the last ones.
+  Blk B;
+  Wt o;
+  auto kstep_and_reload = [&](int blk, auto jc) {
+    kstep(B, o, jc);
+    __builtin_amdgcn_sched_barrier(0);
+    fetch_row(B, blk + WR, decltype(jc)::value);
+  };
+#pragma unroll
+  for (int j = 0; j < 4; ++j) fetch_row(B, w, j);
+  fetch_y(B, w);
+  weights(B, w, o);
+  for (int blk = w; blk < nblk; blk += WR) {
+    fetch_y(B, blk + WR);
+    kstep_and_reload(blk, std::integral_constant<int, 0>{});
+    kstep_and_reload(blk, std::integral_constant<int, 1>{});
+    kstep_and_reload(blk, std::integral_constant<int, 2>{});
+    kstep_and_reload(blk, std::integral_constant<int, 3>{});
+    weights(B, blk + WR, o);
+  }
+}
+
+template <class C, int NB, bool VEC, bool LG>
+__device__ __forceinline__ void gram_pass_nb(Smem<C>& S, const double* X, const double* y, int N, int D, double prior_var,
+                                             const double* vec, double coef, bool want_gv, double& loglik) {
+  constexpr int NTL = NB * (NB + 1) / 2, NTW = (NTL + C::H - 1) / C::H;
+  const int t = threadIdx.x, l = t % 64, w = __builtin_amdgcn_readfirstlane(t / 64);
+  f64x4 acc[NTW];
+#pragma unroll
+  for (int i = 0; i < NTW; ++i) acc[i] = f64x4{0, 0, 0, 0};
+  double ll = 0.0, gacc[NB], gvacc[NB];
+#pragma unroll
+  for (int b = 0; b < NB; ++b) gacc[b] = gvacc[b] = 0.0;
+  if constexpr (C::H == 1) {
+    gram_loop<C, NB, 0, NTW, VEC, LG>(S, X, y, N, D, vec, coef, want_gv, w, acc, ll, gacc, gvacc);
+  } else {
+    // the likelihood and the vector sums belong to the first group
+    if (w < 2) {
+      gram_loop<C, NB, 0, NTW, VEC, LG>(S, X, y, N, D, vec, coef, want_gv, w, acc, ll, gacc, gvacc);
+    } else {
+      gram_loop<C, NB, NTW, NTW, VEC, false>(S, X, y, N, D, vec, coef, false, w - 2, acc, ll, gacc, gvacc);
     }
   }
-  if (want_lg) {
-    S.part[t / C::MAXD][t % C::MAXD] = gacc;
-    loglik = block_sum(S, ll);  // contains the barrier that publishes part[]
-    if (t < D) S.g[t] = column_total(S, t) - S.q[t] / prior_var;
-  }
-  if (want_gv) {
-    __syncthreads();
-    S.part[t / C::MAXD][t % C::MAXD] = gvacc;
-    __syncthreads();
-    if (t < D) S.gv[t] = column_total(S, t) + vec[t] / prior_var;
+  // the partial tiles of a group's waves meet in its first wave, through LDS
+  auto put = [&](double* P) {
+#pragma unroll
+    for (int i = 0; i < NTW; ++i)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) P[(i * 4 + r) * 64 + l] = acc[i][r];
+  };
+  auto add = [&](const double* P) {
+#pragma unroll
+    for (int i = 0; i < NTW; ++i)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) acc[i][r] += P[(i * 4 + r) * 64 + l];
+  };
+  // both triangles of G from lower tiles T0 .., C[4r + l/16][l%16] layout
+  auto store = [&](auto t0c) {
+    constexpr int T0 = decltype(t0c)::value;
+    int i0 = 0;
+#pragma unroll
+    for (int bi = 0; bi < NB; ++bi)
+#pragma unroll
+      for (int bj = 0; bj <= bi; ++bj) {
+        if (i0 >= T0 && i0 < T0 + NTW) {
+#pragma unroll
+          for (int r = 0; r < 4; ++r) {
+            const int i = bi * 16 + 4 * r + l / 16, j = bj * 16 + l % 16;
+            // a diagonal tile holds (i, j) and (j, i) rounded differently: keep the
+            // lower one for both so that G is exactly symmetric
+            if (i < j) continue;
+            const double a = acc[i0 - T0][r];
+            const double v = i == j ? a + 1.0 / prior_var : a;
+            S.Gi[i * C::LDX + j] = v;
+            S.Gi[j * C::LDX + i] = v;
+          }
+        }
+        ++i0;
+      }
+  };
+  if (LG) {
+#pragma unroll
+    for (int b = 0; b < NB; ++b) {
+      const double s = rows_sum(gacc[b]);
+      if (l < 16) S.part[w][16 * b + l] = s;
+    }
   }
   __syncthreads();
+  if constexpr (C::H == 1) {
+    if (w >= 2) put(S.tile + (w - 2) * (NTW * 256));
+    __syncthreads();
+    if (w < 2) add(S.tile + w * (NTW * 256));
+    __syncthreads();
+    if (w == 1) put(S.tile);
+  } else {
+    if (w & 1) put(S.tile + (w / 2) * (NTW * 256));
+  }
+  if (LG && t < D) {
+    double s = 0.0;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) s += S.part[i][t];
+    S.g[t] = s - S.q[t] / prior_var;
+  }
+  __syncthreads();
+  if constexpr (C::H == 1) {
+    if (w == 0) {
+      add(S.tile);
+      store(std::integral_constant<int, 0>{});
+    }
+  } else {
+    if (!(w & 1)) add(S.tile + (w / 2) * (NTW * 256));
+    __syncthreads();  // both groups have read their tiles before G takes the space
+    if (w == 0) store(std::integral_constant<int, 0>{});
+    if (w == 2) store(std::integral_constant<int, NTW>{});
+  }
+  if (VEC && want_gv) {
+#pragma unroll
+    for (int b = 0; b < NB; ++b) {
+      const double s = rows_sum(gvacc[b]);
+      if (l < 16) S.part[w][16 * b + l] = s;
+    }
+  }
+  if (LG) loglik = block_sum(S, ll);
+  __syncthreads();
+  if (VEC && want_gv) {
+    if (t < D) {
+      double s = 0.0;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) s += S.part[i][t];
+      S.gv[t] = s + vec[t] / prior_var;
+    }
+    __syncthreads();
+  }
+}
+
+// want_lg and vec exclude each other.
+template <class C>
+__device__ __forceinline__ void pass_gram(Smem<C>& S, const double* X, const double* y, int N, int D, double prior_var,
+                                          const double* vec, double coef, bool want_lg, bool want_gv, double& loglik) {
+  auto run = [&](auto nbc) __attribute__((always_inline)) {
+    constexpr int NB = decltype(nbc)::value;
+    if (vec != nullptr)
+      gram_pass_nb<C, NB, true, false>(S, X, y, N, D, prior_var, vec, coef, want_gv, loglik);
+    else if (want_lg)
+      gram_pass_nb<C, NB, false, true>(S, X, y, N, D, prior_var, nullptr, 0.0, false, loglik);
+    else
+      gram_pass_nb<C, NB, false, false>(S, X, y, N, D, prior_var, nullptr, 0.0, false, loglik);
+  };
+  by_width<C>(D, run);
 }
 
 template <class C>
@@ -227,65 +404,77 @@ __device__ __forceinline__ void pass1(Smem<C>& S, const double* X, const double*
 
 // Load this lane's BS x BS block of S.Gi into registers (entries past D are 0).
 template <class C>
-__device__ __forceinline__ void load_block(const Smem<C>& S, double (&A)[C::BS][C::BS]) {
+__device__ __forceinline__ void load_block(const Smem<C>& S, double (&A)[C::BS][C::BS], int D) {
   const int t = threadIdx.x;
   const int i0 = C::BS * (t / 16), j0 = C::BS * (t % 16);
 #pragma unroll
   for (int a = 0; a < C::BS; ++a)
 #pragma unroll
-    for (int b = 0; b < C::BS; ++b) A[a][b] = S.Gi[(i0 + a) * C::LDX + j0 + b];
+    for (int b = 0; b < C::BS; ++b) {
+      const double v = S.Gi[(i0 + a) * C::LDX + j0 + b];
+      A[a][b] = (i0 + a < D && j0 + b < D) ? v : 0.0;
+    }
 }
 
-// Symmetric sweep of the first D pivots: A <- -A^-1.  Returns log |det A|.
+// Symmetric sweep of the first D pivots: A <- -A^-1, the pivots to S.dk (their
+// logarithms belong to pivots_logdet: one log per matrix row instead of one
+// in every lane at every pivot).
 // Pivots run in groups of BS with the pivot inside a group unrolled, so the
-// broadcast row k = BS kk + a is register row a of its owners' blocks.
+// broadcast row k = BS kk + a is register row a of its owners' blocks.  Every
+// lane applies a_ij - a_ik a_kj / d; the owners of the pivot column (a_ik / d),
+// the pivot row (a_kj / d) and the pivot (-1/d) then overwrite theirs.
 // With zc != nullptr (A positive definite) it also draws pout = chol(A) zc:
 // at pivot k the unswept part of row k is the Schur complement's column, so
 // L[j][k] = row_k[j] / sqrt(d_k) for j >= k.
 template <class C>
-__device__ __forceinline__ double sweep(Smem<C>& S, double (&A)[C::BS][C::BS], int D, const double* zc = nullptr,
-                        double* pout = nullptr) {
+__device__ __forceinline__ void sweep(Smem<C>& S, double (&A)[C::BS][C::BS], int D, const double* zc = nullptr,
+                                      double* pout = nullptr) {
+  constexpr int BS = C::BS;
   const int t = threadIdx.x;
-  const int i0 = C::BS * (t / 16), j0 = C::BS * (t % 16);
-  double logdet = 0.0;
+  const int i0 = BS * (t / 16), j0 = BS * (t % 16);
   double pacc = 0.0;
-  for (int kk = 0; kk * C::BS < D; ++kk) {
+  for (int kk = 0; kk * BS < D; ++kk) {
+    const bool row = t / 16 == kk, col = t % 16 == kk;
 #pragma unroll
-    for (int a0 = 0; a0 < C::BS; ++a0) {
-      const int k = kk * C::BS + a0;
+    for (int a0 = 0; a0 < BS; ++a0) {
+      const int k = kk * BS + a0;
       if (k >= D) break;
       double* buf = S.rowbuf[k & 1];
-      if (t / 16 == kk) {
+      if (row) {
 #pragma unroll
-        for (int b = 0; b < C::BS; ++b) buf[j0 + b] = A[a0][b];
+        for (int b = 0; b < BS; ++b) buf[j0 + b] = A[a0][b];
       }
       __syncthreads();
       const double d = buf[k];
       const double rd = 1.0 / d;
-      logdet += log(fabs(d));  // log |det|: G +- (eps/2) Omega~ may be indefinite
+      if (t == 0) S.dk[k] = d;
       if (zc != nullptr && t >= k && t < D) pacc = fma(buf[t] * zc[k], 1.0 / sqrt(d), pacc);
-      double bjr[C::BS];
+      double bjr[BS], sc[BS];
 #pragma unroll
-      for (int b = 0; b < C::BS; ++b) bjr[b] = buf[j0 + b] * rd;
-      // branch-free: a_ij - a_ik a_kj / d off the pivot row and column,
-      // a_ik / d on them, -1/d on the pivot
+      for (int b = 0; b < BS; ++b) bjr[b] = buf[j0 + b] * rd;
 #pragma unroll
-      for (int a = 0; a < C::BS; ++a) {
-        const int i = i0 + a;
-        const double aik = buf[i];
+      for (int a = 0; a < BS; ++a) {
+        sc[a] = A[a][a0] * rd;
+        const double aik = buf[i0 + a];
 #pragma unroll
-        for (int b = 0; b < C::BS; ++b) {
-          const int j = j0 + b;
-          const double v = A[a][b];
-          const double upd = fma(-aik, bjr[b], v);
-          const double scaled = v * rd;
-          A[a][b] = (i != k && j != k) ? upd : ((i == k && j == k) ? -rd : scaled);
-        }
+        for (int b = 0; b < BS; ++b) A[a][b] = fma(-aik, bjr[b], A[a][b]);
       }
+#pragma unroll
+      for (int a = 0; a < BS; ++a) A[a][a0] = col ? sc[a] : A[a][a0];
+#pragma unroll
+      for (int b = 0; b < BS; ++b) A[a0][b] = row ? (b == a0 && col ? -rd : bjr[b]) : A[a0][b];
     }
   }
   if (pout != nullptr && t < C::MAXD) pout[t] = t < D ? pacc : 0.0;
-  return logdet;
+}
+
+// log |det A| from the pivots of the last sweep (G +- (eps/2) Omega~ may be
+// indefinite); the same in every lane.
+template <class C>
+__device__ __forceinline__ double pivots_logdet(Smem<C>& S, int D) {
+  __syncthreads();  // the last pivot's write
+  const int t = threadIdx.x;
+  return block_sum(S, t < D ? log(fabs(S.dk[t])) : 0.0);
 }
 
 // Write G^-1 = -A into S.Gi.
@@ -327,97 +516,174 @@ __device__ double cholesky(Smem<C>& S, int D) {
   return logdet;
 }
 
-// u = G^-1 p with G^-1 in S.Gi (vector p in LDS).
+// u = G^-1 p with G^-1 in S.Gi (vector p in LDS): TPR lanes per row.
 // Entries past D are written as zeros: the passes over X multiply whole padded
 // rows by this vector, and 0 times a stale LDS value left by an earlier kernel
 // (possibly Inf or NaN) would not be 0.
 template <class C>
 __device__ __forceinline__ void ginv_times(Smem<C>& S, const double* p, double* out, int D) {
-  const int t = threadIdx.x;
-  if (t < D) {
-    double s = 0.0;
-    for (int j = 0; j < D; ++j) s += S.Gi[t * C::LDX + j] * p[j];
-    out[t] = s;
-  } else if (t < C::MAXD) {
-    out[t] = 0.0;
-  }
+  constexpr int TPR = NT / C::MAXD;
+  const int r = threadIdx.x / TPR, h = threadIdx.x % TPR;
+  double s = 0.0;
+  if (r < D)
+    for (int j = h; j < D; j += TPR) s += S.Gi[r * C::LDX + j] * p[j];
+  s = group_sum<TPR>(s);
+  __syncthreads();  // out may be p
+  if (h == 0) out[r] = r < D ? s : 0.0;
   __syncthreads();
 }
 
 // Quadratic-form pass with G^-1 in S.Gi, a_n = x_n^T G^-1 x_n:
 //   rmhmc = true : S.dH = X^T [ w (a - b^2)/2 - r ] + q / prior_var, b = X S.u
 //   rmhmc = false: S.dH = X^T (w a) = grad log det G.
-template <class C>
-__device__ void pass_quad(Smem<C>& S, const double* X, const double* y, int N, int D, double prior_var, bool rmhmc) {
-  const int t = threadIdx.x, w = t / 64, l = t % 64;
-  const int ksteps = (D + 3) / 4;
-  const int rb = w / C::CB2;          // row block (16 rows) of this wave
-  const int cb0 = 2 * (w % C::CB2);   // first of its two column blocks
-  double dacc = 0.0;
-  for (int n0 = 0; n0 < N; n0 += C::RCH) {
-    load_chunk(S, X, y, N, D, n0);
-    __syncthreads();
-    {
-      const int r = t / C::TPR, c0 = (t % C::TPR) * C::CPT;
-      double eta = 0.0, bq = 0.0;
+//
+// Lane l = 16 g + m holds row n0 + m's features F(s, g) = 8 (s / 2) + 2 g + s % 2
+// (s < 4 NB) of a 16-row block: neighbouring pairs, so that a load brings 16 bytes
+// a lane (8-byte loads of X[n0 + m][4 s + g] kept the address unit busy for longer
+// than the MFMAs: 122 against 103 us a pass, 2 workgroups per CU, 2048 x 64).  K step s
+// of V^T = G^-1 X^T sums over F(s, .); its result slot (t, r) of the lane is the
+// feature of x register 4 t + r (rows of the G^-1 operand permuted alike).  G^-1 is
+// symmetric, so
+// a = sum_t x_t . (2 sum_{t' < t} G^-1_tt' x_t' + G^-1_tt x_t) over 16-feature tiles:
+// 2 NB (NB + 1) MFMAs a block (40 at D = 64) in place of 4 NB^2 (64).  At
+// capacity 64 the operands of G^-1 (2 NB (NB + 1) doubles a lane) stay in registers for
+// the whole pass; at 128 they are read from LDS.
+struct Pair {
+  double v[2];  // 8-byte aligned: a row of odd D starts anywhere
+};
+
+template <class C, int NB, bool RMHMC>
+__device__ __forceinline__ void quad_pass_nb(Smem<C>& S, const double* X, const double* y, int N, int D,
+                                             double prior_var) {
+  constexpr int NS = 4 * NB;
+  constexpr bool REG = C::MAXD == 64;
+  const int t = threadIdx.x, l = t % 64, w = __builtin_amdgcn_readfirstlane(t / 64);
+  const int g = l / 16, m = l % 16;
+  const int nblk = (N + 15) / 16;
+  auto feat = [](int s, int gg) { return 8 * (s / 2) + 2 * gg + s % 2; };
+  // G^-1[feature of row m of tile tt][F(s, g)], s < 4 (tt + 1), read as the transposed element
+  const int rf = feat(m / 4, m % 4);
+  double T[REG ? 2 * NB * (NB + 1) : 1];
+  if constexpr (REG) {
+    int i = 0;
 #pragma unroll
-      for (int e = 0; e < C::CPT; ++e) {
-        const double xv = S.Xs[r * C::LDX + c0 + e];
-        eta += xv * S.q[c0 + e];
-        bq += xv * S.u[c0 + e];
-      }
-      eta = group_sum<C::TPR>(eta);
-      bq = group_sum<C::TPR>(bq);
-      if (t % C::TPR == 0) {
-        const bool ok = n0 + r < N;
-        const double s = sigmoid(eta);
-        S.lam[r] = ok ? s * (1.0 - s) * (1.0 - 2.0 * s) : 0.0;
-        S.rr[r] = ok ? S.yv[r] - s : 0.0;
-        S.bb[r] = bq;
-      }
-    }
-    // V = X_chunk G^-1 on MFMA: this wave's 16 rows x 32 columns
-    f64x4 v[2] = {f64x4{0, 0, 0, 0}, f64x4{0, 0, 0, 0}};
-    for (int ks = 0; ks < ksteps; ++ks) {
-      const double af = S.Xs[(rb * 16 + l % 16) * C::LDX + ks * 4 + l / 16];
+    for (int tt = 0; tt < NB; ++tt)
 #pragma unroll
-      for (int c = 0; c < 2; ++c) {
-        const double bf = S.Gi[(ks * 4 + l / 16) * C::LDX + (cb0 + c) * 16 + l % 16];
-        v[c] = __builtin_amdgcn_mfma_f64_16x16x4f64(af, bf, v[c], 0, 0, 0);
-      }
-    }
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int row = rb * 16 + 4 * r + l / 16;
-      double s = 0.0;
-#pragma unroll
-      for (int c = 0; c < 2; ++c) s += v[c][r] * S.Xs[row * C::LDX + (cb0 + c) * 16 + l % 16];
-      s = group_sum<16>(s);
-      if (l % 16 == 0) S.aa[w % C::CB2][row] = s;
-    }
-    __syncthreads();
-    if (t < C::RCH) {
-      double a = 0.0;
-#pragma unroll
-      for (int s = 0; s < C::CB2; ++s) a += S.aa[s][t];
-      const double b = S.bb[t];
-      S.hh[t] = rmhmc ? 0.5 * S.lam[t] * (a - b * b) - S.rr[t] : S.lam[t] * a;
-    }
-    __syncthreads();
-    {
-      const int k = t % C::MAXD;
-#pragma unroll
-      for (int m = 0; m < C::RCH / C::RG; ++m) {
-        const int r = t / C::MAXD + C::RG * m;
-        dacc += S.Xs[r * C::LDX + k] * S.hh[r];
-      }
-    }
-    __syncthreads();
+      for (int s = 0; s < 4 * (tt + 1); ++s) T[i++] = S.Gi[feat(s, g) * C::LDX + 16 * tt + rf];
   }
-  S.part[t / C::MAXD][t % C::MAXD] = dacc;
+  double dacc[NS];
+#pragma unroll
+  for (int s = 0; s < NS; ++s) dacc[s] = 0.0;
+  // features past D read feature D - 1 and rows past N row N - 1 (in bounds;
+  // they meet zeros of G^-1, q and u, or a weight of zero)
+  // (byte offsets from a block's first row, as in gram_loop)
+  uint32_t lastb[4];
+#pragma unroll
+  for (int s = 0; s < 4; ++s) lastb[s] = 8u * (uint32_t)min(16 * (NB - 1) + feat(s, g), D - 1);
+  const uint32_t rowb = 8u * (uint32_t)(m * D), gb = 16u * (uint32_t)g;
+  auto fetch = [&](auto whole, double (&x)[NS], double& yv, int blk) {
+    const int n0 = 16 * min(blk, nblk - 1);
+    const char* const Xb = reinterpret_cast<const char*>(X + (size_t)n0 * D);
+    const uint32_t row = min(rowb, 8u * (uint32_t)(min(N - n0 - 1, 15) * D));
+    const Pair* const xr = reinterpret_cast<const Pair*>(Xb + (row + gb));
+#pragma unroll
+    for (int s = 0; s < NS - 4; s += 2) {
+      const Pair p = xr[2 * s];
+      x[s] = p.v[0];
+      x[s + 1] = p.v[1];
+    }
+    if (whole) {
+#pragma unroll
+      for (int s = NS - 4; s < NS; s += 2) {
+        const Pair p = xr[2 * s];
+        x[s] = p.v[0];
+        x[s + 1] = p.v[1];
+      }
+    } else {
+#pragma unroll
+      for (int s = 0; s < 4; ++s) x[NS - 4 + s] = *reinterpret_cast<const double*>(Xb + (row + lastb[s]));
+    }
+    yv = (y + n0)[min(m, N - n0 - 1)];
+  };
+  auto block = [&](const double (&x)[NS], double yv, int blk) {
+    asm volatile("" ::: "memory");  // q and u (at 128 G^-1 too) are read from LDS per block, not held
+    double eta = 0.0, b = 0.0;
+#pragma unroll
+    for (int s = 0; s < NS; ++s) {
+      eta = fma(x[s], S.q[feat(s, g)], eta);
+      if constexpr (RMHMC) b = fma(x[s], S.u[feat(s, g)], b);
+    }
+    eta = rows_sum(eta);
+    if constexpr (RMHMC) b = rows_sum(b);
+    double a = 0.0;
+    int i = 0;
+#pragma unroll
+    for (int tt = 0; tt < NB; ++tt) {
+      f64x4 v = f64x4{0, 0, 0, 0};
+#pragma unroll
+      for (int s = 0; s < 4 * (tt + 1); ++s) {
+        if (s == 4 * tt && tt > 0) v *= 2.0;
+        const double gi = REG ? T[REG ? i : 0] : S.Gi[feat(s, g) * C::LDX + 16 * tt + rf];
+        ++i;
+        v = __builtin_amdgcn_mfma_f64_16x16x4f64(gi, x[s], v, 0, 0, 0);
+      }
+#pragma unroll
+      for (int r = 0; r < 4; ++r) a = fma(v[r], x[4 * tt + r], a);
+    }
+    a = rows_sum(a);
+    const bool ok = 16 * blk + m < N;
+    const double s = sigmoid(eta);
+    const double wv = s * (1.0 - s) * (1.0 - 2.0 * s);
+    const double hv = RMHMC ? 0.5 * wv * (a - b * b) - (yv - s) : wv * a;
+    const double h = ok ? hv : 0.0;
+#pragma unroll
+    for (int s2 = 0; s2 < NS; ++s2) dacc[s2] = fma(x[s2], h, dacc[s2]);
+  };
+  // two register sets in turn (loads one block ahead: with one set, refilled at
+  // the block's end, a pass took 235 us in place of 122)
+  auto loop = [&](auto whole) {
+    double x0[NS], x1[NS], y0, y1;
+    if (nblk > 0) fetch(whole, x0, y0, w);
+    for (int blk = w; blk < nblk; blk += 8) {
+      fetch(whole, x1, y1, blk + 4);
+      block(x0, y0, blk);
+      fetch(whole, x0, y0, blk + 8);
+      if (blk + 4 < nblk) block(x1, y1, blk + 4);
+    }
+  };
+  // a loop of its own for whole tiles keeps the body one basic block (110 -> 101 us);
+  // at capacity 128 it spills (189 -> 240 us): there the choice stays inside
+  if constexpr (!REG)
+    loop(D == 16 * NB);
+  else if (D == 16 * NB)
+    loop(std::true_type{});
+  else
+    loop(std::false_type{});
+#pragma unroll
+  for (int s = 0; s < NS; ++s) {
+    const double v = group_sum<16>(dacc[s]);
+    if (m == 0) S.part[w][feat(s, g)] = v;
+  }
   __syncthreads();
-  if (t < D) S.dH[t] = column_total(S, t) + (rmhmc ? S.q[t] / prior_var : 0.0);
+  if (t < D) {
+    double s = 0.0;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) s += S.part[i][t];
+    S.dH[t] = s + (RMHMC ? S.q[t] / prior_var : 0.0);
+  }
   __syncthreads();
+}
+
+template <class C>
+__device__ __forceinline__ void pass_quad(Smem<C>& S, const double* X, const double* y, int N, int D, double prior_var,
+                                          bool rmhmc) {
+  by_width<C>(D, [&](auto nbc) __attribute__((always_inline)) {
+    constexpr int NB = decltype(nbc)::value;
+    if (rmhmc)
+      quad_pass_nb<C, NB, true>(S, X, y, N, D, prior_var);
+    else
+      quad_pass_nb<C, NB, false>(S, X, y, N, D, prior_var);
+  });
 }
 
 template <class C>

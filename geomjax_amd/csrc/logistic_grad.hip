@@ -43,7 +43,40 @@
 namespace gjx {
 namespace lgrad {
 
-using namespace logistic;
+using logistic::f64x4;
+using logistic::NT;
+using logistic::sigmoid;
+using logistic::softplus;
+
+// Feature capacity MD.  The passes stage X in LDS chunks of RCH rows: TPR lanes
+// per row in the per-row passes (CPT = 8 columns each), the NLT lower Gram tiles
+// dealt to the waves (TPW each at most), RG row groups of the column-per-lane
+// accumulations.
+template <int MD>
+struct Cfg {
+  static_assert(MD == 64 || MD == 128, "feature capacity 64 or 128");
+  static constexpr int MAXD = MD;
+  static constexpr int RCH = MD == 64 ? 32 : 16;
+  static constexpr int LDX = MD + 1;
+  static constexpr int TB = MD / 16;
+  static constexpr int NLT = TB * (TB + 1) / 2;
+  static constexpr int TPW = (NLT + 3) / 4;
+  static constexpr int BS = MD / 16;
+  static constexpr int TPR = NT / RCH;
+  static constexpr int CPT = MD / TPR;
+  static constexpr int RG = NT / MD;
+  static constexpr int CB2 = TB / 2;          // column-block pairs of the quadratic-form pass
+  static constexpr int RB = RCH / 16;         // 16-row blocks per chunk
+  static_assert(RB * CB2 == 4, "the quadratic-form pass gives each wave one (row block, column pair)");
+};
+
+// the lower-triangular 16 x 16 tiles (bi >= bj) in the order (0,0),(1,0),(1,1),(2,0),...
+__device__ __forceinline__ void tile_of(int t, int& bi, int& bj) {
+  int i = 0;
+  while ((i + 1) * (i + 2) / 2 <= t) ++i;
+  bi = i;
+  bj = t - i * (i + 1) / 2;
+}
 
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 
@@ -602,11 +635,11 @@ hipError_t launch_tangent(const LogisticArgs& a, const TangentOut& o, hipStream_
 }  // namespace lgrad
 
 hipError_t launch_logistic_rmhmc_tangent(const LogisticArgs& a, const TangentOut& o, hipStream_t stream) {
-  return lgrad::launch_tangent<double, logistic::Cfg<64>>(a, o, stream);
+  return lgrad::launch_tangent<double, lgrad::Cfg<64>>(a, o, stream);
 }
 
 hipError_t launch_logistic_rmhmc_tangent_f32_wide(const LogisticArgs& a, const TangentOut& o, hipStream_t stream) {
-  return lgrad::launch_tangent<float, logistic::Cfg<128>>(a, o, stream);
+  return lgrad::launch_tangent<float, lgrad::Cfg<128>>(a, o, stream);
 }
 
 }  // namespace gjx

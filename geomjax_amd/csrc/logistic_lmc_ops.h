@@ -23,7 +23,7 @@ __device__ __forceinline__ double lmc_position_pass(Smem<C64>& S, double (&A)[4]
   constexpr int MAXD = C64::MAXD, LDX = C64::LDX;
   const int t = threadIdx.x;
   pass_gram(S, X, y, N, D, prior, nullptr, 0.0, true, false, loglik);
-  load_block(S, A);
+  load_block(S, A, D);
   __syncthreads();
   if (chol_draw) {
     cholesky(S, D);
@@ -36,8 +36,8 @@ __device__ __forceinline__ double lmc_position_pass(Smem<C64>& S, double (&A)[4]
       __syncthreads();
     }
   }
-  const double ld = sweep(S, A, D);
-  __syncthreads();
+  sweep(S, A, D);
+  const double ld = pivots_logdet(S, D);
   store_neg_block(S, A);
   __syncthreads();
   pass_quad(S, X, y, N, D, prior, false);  // S.dH = X^T (w a)
@@ -60,10 +60,10 @@ __device__ __forceinline__ void lmc_half_step(Smem<C64>& S, double (&A)[4][4], c
   __syncthreads();
   // A+ = G + (eps/2) Omega~(v) and G v
   pass_gram(S, X, y, N, D, prior, S.p, 0.25 * eps, false, true, dd);
-  load_block(S, A);
+  load_block(S, A, D);
   __syncthreads();
-  dJ -= sweep(S, A, D);
-  __syncthreads();
+  sweep(S, A, D);
+  dJ -= pivots_logdet(S, D);
   store_neg_block(S, A);  // S.Gi = A+^-1
   // v_temp = G v - (eps/2) (-g + grad log det G / 2)
   if (t < D) S.qs[t] = S.gv[t] - 0.5 * eps * (-S.u[t] + 0.5 * S.vt[t]);
@@ -71,10 +71,10 @@ __device__ __forceinline__ void lmc_half_step(Smem<C64>& S, double (&A)[4][4], c
   ginv_times(S, S.qs, S.p, D);  // v' = A+^-1 v_temp
   // A- = G - (eps/2) Omega~(v')
   pass_gram(S, X, y, N, D, prior, S.p, -0.25 * eps, false, false, dd);
-  load_block(S, A);
+  load_block(S, A, D);
   __syncthreads();
-  dJ += sweep(S, A, D);
-  __syncthreads();
+  sweep(S, A, D);
+  dJ += pivots_logdet(S, D);
   if (t < D) {
     S.g[t] = S.u[t];
     S.dH[t] = S.vt[t];

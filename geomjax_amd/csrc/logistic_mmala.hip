@@ -57,10 +57,10 @@ __device__ __forceinline__ double mmala_position(Smem<C64>& S, double (&A)[4][4]
                                                  double& loglik) {
   pass_gram(S, X, y, N, D, prior, nullptr, 0.0, true, false, loglik);
   if (metric_dst != nullptr) write_metric(S, metric_dst, D, Dp);
-  load_block(S, A);
+  load_block(S, A, D);
   __syncthreads();
-  const double ld = sweep(S, A, D);
-  __syncthreads();
+  sweep(S, A, D);
+  const double ld = pivots_logdet(S, D);
   store_neg_block(S, A);
   __syncthreads();
   pass_quad(S, X, y, N, D, prior, false);
@@ -175,9 +175,9 @@ __global__ void __launch_bounds__(NT, 2) logistic_mmala_f64_kernel(const Logisti
     const double gamma0 = drift(S, D);
     const double mu = own ? S.q0[t] + eps * S.u[t] : 0.0;
     // chol(G^-1) z by a sweep over G^-1 (the inverse itself stays in S.Gi)
-    load_block(S, A);
+    load_block(S, A, D);
     __syncthreads();
-    (void)sweep(S, A, D, S.z, S.p);
+    sweep(S, A, D, S.z, S.p);
     __syncthreads();
     const double x1 = own ? mu + sq2e * S.p[t] : 0.0;
     const double zz = block_sum(S, own ? S.z[t] * S.z[t] : 0.0);

@@ -303,10 +303,10 @@ __global__ void __launch_bounds__(NT, 1) logistic_nuts_f64_kernel(const Logistic
   double dummy = 0.0;
   pass1(S, X, y, N, D, prior, false, dummy);
   double A[BS][BS];
-  load_block(S, A);
+  load_block(S, A, D);
   __syncthreads();
-  const double logdet = sweep(S, A, D, S.z, S.p0);
-  __syncthreads();
+  sweep(S, A, D, S.z, S.p0);
+  const double logdet = pivots_logdet(S, D);
   if (t < MAXD) S.p[t] = S.p0[t];
   if (a.momentum != nullptr && own) static_cast<double*>(a.momentum)[(size_t)c * a.Dmax + t] = S.p0[t];
   store_neg_block(S, A);
@@ -320,7 +320,7 @@ __global__ void __launch_bounds__(NT, 1) logistic_nuts_f64_kernel(const Logistic
     if (!have_ginv) {
       double dd = 0.0;
       pass1(S, X, y, N, D, prior, false, dd);
-      load_block(S, A);
+      load_block(S, A, D);
       __syncthreads();
       sweep(S, A, D);
       __syncthreads();
@@ -336,22 +336,19 @@ __global__ void __launch_bounds__(NT, 1) logistic_nuts_f64_kernel(const Logistic
   auto step = [&](double hstep, Pt& out) -> double {
     const double h = 0.5 * hstep;
     const double q0v = t < MAXD ? S.q[t] : 0.0, p0v = t < MAXD ? S.p[t] : 0.0;
-    feval();  // first evaluation outside the loop (integrators.py:84)
-    double norm;
-    {
-      double dq = 0.0;
-      if (own) {
-        const double qn = q0v + h * S.u[t];
-        const double pn = p0v - h * S.dH[t];
-        dq = nan_max(fabs(qn - S.q[t]), fabs(pn - S.p[t]));
-        S.q[t] = qn;
-        S.p[t] = pn;
-      }
-      norm = block_max(S, dq);
-    }
-    int n = 0;
-    while (n < a.max_iters && isfinite(norm) && norm < a.div_tol && norm > a.conv_tol) {
+    // the first evaluation (integrators.py:84) is outside the loop count; the
+    // last one is the explicit half step from the last iterate (:146-148)
+    int n = -1;
+    for (bool last = false;;) {
       feval();
+      if (last) {
+        if (own) {
+          S.q[t] = S.q[t] + h * S.u[t];
+          S.p[t] = S.p[t] - h * S.dH[t];
+        }
+        __syncthreads();
+        break;
+      }
       double dq = 0.0;
       if (own) {
         const double qn = q0v + h * S.u[t];
@@ -360,22 +357,16 @@ __global__ void __launch_bounds__(NT, 1) logistic_nuts_f64_kernel(const Logistic
         S.q[t] = qn;
         S.p[t] = pn;
       }
-      norm = block_max(S, dq);
+      const double norm = block_max(S, dq);
       ++n;
+      last = !(n < a.max_iters && isfinite(norm) && norm < a.div_tol && norm > a.conv_tol);
     }
-    // explicit half step from the last iterate (integrators.py:146-148)
-    feval();
-    if (own) {
-      S.q[t] = S.q[t] + h * S.u[t];
-      S.p[t] = S.p[t] - h * S.dH[t];
-    }
-    __syncthreads();
     double loglik = 0.0;
     pass1(S, X, y, N, D, prior, true, loglik);
-    load_block(S, A);
+    load_block(S, A, D);
     __syncthreads();
-    const double ld = sweep(S, A, D);
-    __syncthreads();
+    sweep(S, A, D);
+    const double ld = pivots_logdet(S, D);
     store_neg_block(S, A);
     __syncthreads();
     ginv_times(S, S.p, S.u, D);

@@ -17,15 +17,15 @@
 //
 // One workgroup (256 lanes, 4 waves) owns one chain for the whole launch, so
 // every chain runs its own fixed-point iteration count.  Two instantiations by
-// feature capacity: 64 (X in LDS chunks of 32 rows, 10 lower 16x16 Gram tiles,
-// 4x4 inverse entries per lane) and 128 (chunks of 16 rows, 36 tiles, 8x8
-// entries per lane; G^-1 alone is 129 KiB of LDS).  Per evaluation:
-//   pass 1: eta = X q, lambda, and the Gram X^T diag(lambda) X on MFMA
-//           (lower tiles owned by waves);
+// feature capacity: 64 (10 lower 16x16 Gram tiles, 4x4 inverse entries per
+// lane) and 128 (36 tiles, 8x8 entries per lane; G^-1 alone is 129 KiB of LDS).
+// Per evaluation (logistic_common.h):
+//   pass 1: eta = X q, lambda, and the Gram X^T diag(lambda) X on MFMA (rows of X
+//           dealt to the waves);
 //   sweep : G^-1 by the symmetric sweep operator with G held in registers
 //           (one barrier per pivot), log det G = sum of the pivots' logs;
-//   pass 2: eta, s, w, r, b = X u on VALU, V = X_chunk G^-1 on MFMA,
-//           a_n = x_n . V_n, h_n, and X^T h.
+//   pass 2: eta, s, w, r, b = X u on VALU, V = X G^-1 on MFMA (the lower tiles,
+//           G^-1 being symmetric), a_n = x_n . V_n, h_n, and X^T h.
 // The momentum draw p0 = chol(G) z comes out of the first sweep of each
 // transition: before pivot k is eliminated, row k of the partly swept matrix
 // holds column k of the Schur complement, i.e. sqrt(d_k) L[:, k].
@@ -101,11 +101,11 @@ __global__ void __launch_bounds__(NT, MD == 64 ? 2 : 1) logistic_rmhmc_f64_kerne
     double dummy = 0.0;
     pass1(S, X, y, N, D, prior, false, dummy);
     double A[BS][BS];
-    load_block(S, A);
+    load_block(S, A, D);
     __syncthreads();
     // the sweep also draws p0 = chol(G(q0)) z from its Schur-complement columns
-    double logdet = sweep(S, A, D, S.z, S.p0);
-    __syncthreads();
+    sweep(S, A, D, S.z, S.p0);
+    double logdet = pivots_logdet(S, D);
     if (t < MAXD) S.p[t] = S.p0[t];
     if (STEP && a.momentum != nullptr && t < D) static_cast<double*>(a.momentum)[(size_t)c * Dp + t] = S.p0[t];
     store_neg_block(S, A);
@@ -123,7 +123,7 @@ __global__ void __launch_bounds__(NT, MD == 64 ? 2 : 1) logistic_rmhmc_f64_kerne
       if (!have_ginv) {
         double dd = 0.0;
         pass1(S, X, y, N, D, prior, false, dd);
-        load_block(S, A);
+        load_block(S, A, D);
         __syncthreads();
         sweep(S, A, D);
         __syncthreads();
@@ -145,23 +145,20 @@ __global__ void __launch_bounds__(NT, MD == 64 ? 2 : 1) logistic_rmhmc_f64_kerne
         q0v = S.q[t];
         p0v = S.p[t];
       }
-      // first evaluation outside the loop (integrators.py:84)
-      feval();
-      double norm;
-      {
-        double dq = 0.0;
-        if (t < D) {
-          const double qn = q0v + h * S.u[t];
-          const double pn = p0v - h * S.dH[t];
-          dq = nan_max(fabs(qn - S.q[t]), fabs(pn - S.p[t]));
-          S.q[t] = qn;
-          S.p[t] = pn;
-        }
-        norm = block_max(S, dq);
-      }
-      int n = 0;
-      while (n < a.max_iters && isfinite(norm) && norm < a.div_tol && norm > a.conv_tol) {
+      // the first evaluation (integrators.py:84) is outside the loop count; the
+      // last one is the explicit half step from the last iterate (:146-148).  One
+      // call site: the passes are inlined once.
+      int n = -1;
+      for (bool last = false;;) {
         feval();
+        if (last) {
+          if (t < D) {
+            S.q[t] = S.q[t] + h * S.u[t];
+            S.p[t] = S.p[t] - h * S.dH[t];
+          }
+          __syncthreads();
+          break;
+        }
         double dq = 0.0;
         if (t < D) {
           const double qn = q0v + h * S.u[t];
@@ -170,31 +167,25 @@ __global__ void __launch_bounds__(NT, MD == 64 ? 2 : 1) logistic_rmhmc_f64_kerne
           S.q[t] = qn;
           S.p[t] = pn;
         }
-        norm = block_max(S, dq);
+        const double norm = block_max(S, dq);
         ++n;
+        last = !(n < a.max_iters && isfinite(norm) && norm < a.div_tol && norm > a.conv_tol);
+        if (STEP && last && t == 0) {
+          const size_t idx = (size_t)c * a.L + s;
+          if (a.fp_iters) a.fp_iters[idx] = n;
+          if (a.fp_norm) a.fp_norm[idx] = norm;
+          if (a.fp_success) a.fp_success[idx] = (uint8_t)(isfinite(norm) && norm <= a.conv_tol);
+        }
       }
-      if (STEP && t == 0) {
-        const size_t idx = (size_t)c * a.L + s;
-        if (a.fp_iters) a.fp_iters[idx] = n;
-        if (a.fp_norm) a.fp_norm[idx] = norm;
-        if (a.fp_success) a.fp_success[idx] = (uint8_t)(isfinite(norm) && norm <= a.conv_tol);
-      }
-      // explicit half step from the last iterate (integrators.py:146-148)
-      feval();
-      if (t < D) {
-        S.q[t] = S.q[t] + h * S.u[t];
-        S.p[t] = S.p[t] - h * S.dH[t];
-      }
-      __syncthreads();
     }
 
     // ---- end: l, grad l, G^-1, velocity and energy at (q_L, p_L) ----
     double loglik = 0.0;
     pass1(S, X, y, N, D, prior, true, loglik);  // S.g = grad l(q_L)
-    load_block(S, A);
+    load_block(S, A, D);
     __syncthreads();
-    logdet = sweep(S, A, D);
-    __syncthreads();
+    sweep(S, A, D);
+    logdet = pivots_logdet(S, D);
     store_neg_block(S, A);
     __syncthreads();
     ginv_times(S, S.p, S.u, D);
