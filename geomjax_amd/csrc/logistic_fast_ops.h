@@ -67,6 +67,32 @@ __device__ __forceinline__ void wave0_sync() {
 // arithmetic on it stays scalar).
 __device__ __forceinline__ int wave_id() { return __builtin_amdgcn_readfirstlane((int)threadIdx.x / 64); }
 
+// The lane's index as a value that the compiler cannot trace back to threadIdx: a
+// pass's lane-dependent addresses are formed where the pass starts.  Known to be
+// loop invariant they are hoisted above the kernel's stage loop, and the dozens of
+// them, live through every pass, are spilled inside the passes' loops.
+__device__ __forceinline__ int pass_lane() {
+  int l = (int)threadIdx.x % 64;
+  asm volatile("" : "+v"(l));
+  return l;
+}
+
+// p + off bytes for a uniform p and a 32-bit lane offset: loads and stores keep p
+// in scalar registers (an index of the element type is widened into a 64-bit vector
+// address per access: two registers and an instruction each)
+template <class T>
+__device__ __forceinline__ T* at_byte(T* p, uint32_t off) {
+  using C = std::conditional_t<std::is_const_v<T>, const char, char>;
+  return reinterpret_cast<T*>(reinterpret_cast<C*>(p) + off);
+}
+
+// A lane offset for at_byte inside a loop: opaque, so that it is widened next to the
+// loads (where it folds into them) and not once before the loop
+__device__ __forceinline__ uint32_t here(uint32_t off) {
+  asm volatile("" : "+v"(off));
+  return off;
+}
+
 // Sum of one value per wave, identical in every wave (LDS scratch S.red).
 template <int NW>
 __device__ __forceinline__ double waves_sum(Smem<NW>& S, double v) {
@@ -115,12 +141,11 @@ template <int NB, int NW, bool SIGNED = false>
 __device__ __forceinline__ void gram_pass(Smem<NW>& S, const float* __restrict__ Xg, const float* __restrict__ sl, int npad, int D,
                           float inv_prior) {
   constexpr int NTL = NB * (NB + 1) / 2;
-  const int l = threadIdx.x % 64, w = wave_id();
+  const int l = pass_lane(), w = wave_id();
   f32x16 acc[NTL];
 #pragma unroll
   for (int t = 0; t < NTL; ++t) acc[t] = f32x16{0};
-  const float* slp = sl + (l / 32) * 8;
-  const float* xp = Xg + (size_t)l * 8;
+  const uint32_t so = 32u * (uint32_t)(l / 32), xo = 32u * (uint32_t)l;
   const int nj = 4 * own_groups<NW>(npad, w);  // this wave's K steps (none for a wave without rows)
   // fragments of K step kb: sqrt(lambda) of the lane's 8 rows and X of its NB feature blocks
   struct Frag {
@@ -131,9 +156,10 @@ __device__ __forceinline__ void gram_pass(Smem<NW>& S, const float* __restrict__
     // the pipeline's tail re-reads the wave's last step (in bounds, unused)
     const int jj = j < nj ? j : nj - 1;
     const int kb = jj >= 0 ? own_kstep<NW>(jj, w) : 0;
-    load8(slp + kb * 16, f.s);
+    load8(at_byte(sl + kb * 16, here(so)), f.s);
+    const uint32_t o = here(xo);
 #pragma unroll
-    for (int b = 0; b < NB; ++b) load8(xp + (size_t)(kb * NB + b) * 512, f.x[b]);
+    for (int b = 0; b < NB; ++b) load8(at_byte(Xg + (size_t)(kb * NB + b) * 512, o), f.x[b]);
   };
   auto split_frag = [&](const Frag& f, bf16x8 (&hi)[NB], bf16x8 (&lo)[NB], uint32_t (&m)[4]) {
 #pragma unroll
@@ -172,10 +198,17 @@ __device__ __forceinline__ void gram_pass(Smem<NW>& S, const float* __restrict__
   Frag f0, f1, f2, f3;
   bf16x8 ha[NB], la[NB], hb[NB], lb[NB];
   uint32_t ma[4], mb[4];  // row signs (SIGNED only)
+  // The prologue's loads keep the loop's order (the barriers): a wait in the loop
+  // is sized for the worse of the two orders that reach it, and with these loads
+  // reordered the first wait of every iteration asked for all but the newest step.
   fetch(f0, 0);
+  __builtin_amdgcn_sched_barrier(0);
   fetch(f1, 1);
+  __builtin_amdgcn_sched_barrier(0);
   fetch(f2, 2);
+  __builtin_amdgcn_sched_barrier(0);
   fetch(f3, 3);
+  __builtin_amdgcn_sched_barrier(0);
   split_frag(f0, ha, la, ma);
   for (int j = 0; j < nj; j += 4) {
     fetch(f0, j + 4);
@@ -248,7 +281,7 @@ template <int NB, int NW>
 __device__ __forceinline__ void sweep(Smem<NW>& S, f32x32 (&A)[NB], int D, bool want_chol, float& p0j,
                                       bool store_l = false) {
   constexpr int DP = 32 * NB;
-  const int jl = threadIdx.x % DP;
+  const int jl = pass_lane() % DP;
 #pragma unroll
   for (int b = 0; b < NB; ++b)
 #pragma unroll
@@ -324,7 +357,7 @@ template <int NB, int NW>
 __device__ __forceinline__ void solve_refined(Smem<NW>& S, const f32x32 (&A)[NB], const float* rhs, float* out,
                                               float* tmp) {
   constexpr int DP = 32 * NB;
-  const int l = threadIdx.x, jl = l % DP;
+  const int l = pass_lane(), jl = l % DP;  // (runs on the first wave)
   float uj = 0.0f;
 #pragma unroll
   for (int b = 0; b < NB; ++b)
@@ -352,7 +385,7 @@ __device__ __forceinline__ void solve_refined(Smem<NW>& S, const f32x32 (&A)[NB]
 template <int NB, int NW>
 __device__ __forceinline__ void ginv_apply(Smem<NW>& S, const f32x32 (&A)[NB]) {
   constexpr int DP = 32 * NB;
-  const int l = threadIdx.x, jl = l % DP;
+  const int l = pass_lane(), jl = l % DP;  // (runs on the first wave)
   float uj = 0.0f;
 #pragma unroll
   for (int b = 0; b < NB; ++b)
@@ -378,7 +411,7 @@ __device__ __forceinline__ void ginv_apply(Smem<NW>& S, const f32x32 (&A)[NB]) {
 // G^-1 into its buffer (over G with one wave per chain: call after the last read of G)
 template <int NB, int NW>
 __device__ __forceinline__ void store_ginv(Smem<NW>& S, const f32x32 (&A)[NB]) {
-  const int l = threadIdx.x;
+  const int l = pass_lane();  // (runs on the first wave)
   if (l < 32 * NB) {
 #pragma unroll
     for (int b = 0; b < NB; ++b)
@@ -413,7 +446,7 @@ template <int NB, int NW>
 __device__ __forceinline__ float reduce_features(Smem<NW>& S, const float (&acc)[2 * NB][8]) {
   constexpr int KC = 2 * NB, RS = KC * 8 + 1;
   static_assert(NW * 64 * RS <= MAXD * LDG, "the partials must fit S.G");
-  const int t = threadIdx.x, l = t % 64;
+  const int l = pass_lane(), t = 64 * wave_id() + l;
   float* R = S.G;  // no Gram is live during a row pass, and G^-1 is no longer read
   __syncthreads();
 #pragma unroll
@@ -439,6 +472,18 @@ __device__ __forceinline__ float reduce_features(Smem<NW>& S, const float (&acc)
 // the explicit half step, which also sets E0), SL <- sqrt(lambda) there.
 // ---------------------------------------------------------------------------
 //
+// G^-1 is symmetric, so with 32-feature tiles
+//   a_n = sum_t x_t . (2 sum_{t' < t} G^-1_tt' x_t' + G^-1_tt x_t):
+// only the products of its lower tiles are formed, the off-diagonal ones from
+// the doubled entries (exact): NB (NB + 1) fragment products a block (6 at 64
+// features, 8 for all of V^T).  At 2048 x 64 an evaluation of 1024 resident chains went
+// from 128 to 118 us, of 2048 from 220 to 208 (there the rows' way from L2 and VALU
+// issue bound it as much: with these MFMAs alone taken out it does not change).
+// Measured and not kept: rows split into bf16 pairs here instead of loaded
+// (half the bytes, 96 more VALU instructions a block: 208 -> 230 us), row scalars loaded
+// two blocks ahead (no change), packed fragments a lane-contiguous 16 bytes at
+// a time (no change).
+//
 // The A operand (rows of G^-1 permuted by phi, split) is staged once in LDS
 // over S.G, which is not read again before the next Gram pass rewrites it
 // (with one wave per chain G^-1 itself lives there: every wave reads its share
@@ -449,29 +494,37 @@ template <int NB, int NW>
 __device__ __forceinline__ void field_pass(Smem<NW>& S, const float* __restrict__ Xr, const float* __restrict__ Xs,
                                            const float* __restrict__ yf, float* E0, float* E1, float* SL, int npad,
                                            int D, float hs, float inv_prior, bool explicit_step) {
-  constexpr int KC = 2 * NB, NTK = NB * KC, PER = (NTK + NW - 1) / NW;
-  const int t = threadIdx.x, l = t % 64, w = wave_id(), h = l / 32;
-  bf16x8* const AH = reinterpret_cast<bf16x8*>(S.G);  // [NTK][64 lanes]
-  bf16x8* const AL = AH + NTK * 64;
-  static_assert(2 * NTK * 64 * sizeof(bf16x8) <= sizeof(S.G), "the split G^-1 operand must fit S.G");
+  constexpr int KC = 2 * NB, NF = NB * (NB + 1);
+  const int l = pass_lane(), w = wave_id(), t = 64 * w + l, h = l / 32;
+  bf16x8* const AH = reinterpret_cast<bf16x8*>(S.G);  // [NF][64 lanes], in the order of the products
+  bf16x8* const AL = AH + NF * 64;
+  static_assert(2 * NF * 64 * sizeof(bf16x8) <= sizeof(S.G), "the split G^-1 operand must fit S.G");
   {
-    float v[PER][8];
+    float v[NF][8];
+    int f = 0;
 #pragma unroll
-    for (int j = 0; j < PER; ++j) {
-      const int tk = w + NW * j;
-      if (tk < NTK) load8(S.gi() + phi((tk / KC) * 32 + (l % 32)) * LDG + (tk % KC) * 16 + h * 8, v[j]);
-    }
-    __syncthreads();
+    for (int kc = 0; kc < KC; ++kc)
 #pragma unroll
-    for (int j = 0; j < PER; ++j) {
-      const int tk = w + NW * j;
-      if (tk < NTK) {
-        bf16x8 hi, lo;
-        split8(v[j], hi, lo);
-        AH[tk * 64 + l] = hi;
-        AL[tk * 64 + l] = lo;
+      for (int tt = kc / 2; tt < NB; ++tt) {
+        if (f % NW == w) load8(S.gi() + phi(tt * 32 + (l % 32)) * LDG + kc * 16 + h * 8, v[f]);
+        ++f;
       }
-    }
+    __syncthreads();
+    f = 0;
+#pragma unroll
+    for (int kc = 0; kc < KC; ++kc)
+#pragma unroll
+      for (int tt = kc / 2; tt < NB; ++tt) {
+        if (f % NW == w) {
+#pragma unroll
+          for (int i = 0; i < 8; ++i) v[f][i] *= tt > kc / 2 ? 2.0f : 1.0f;
+          bf16x8 hi, lo;
+          split8(v[f], hi, lo);
+          AH[f * 64 + l] = hi;
+          AL[f * 64 + l] = lo;
+        }
+        ++f;
+      }
   }
   __syncthreads();
   float dacc[KC][8];
@@ -479,9 +532,8 @@ __device__ __forceinline__ void field_pass(Smem<NW>& S, const float* __restrict_
   for (int kc = 0; kc < KC; ++kc)
 #pragma unroll
     for (int i = 0; i < 8; ++i) dacc[kc][i] = 0.0f;
-  const uint32_t xoff = (uint32_t)l * 8u;
+  const uint32_t xo = 32u * (uint32_t)l, ro = 4u * (uint32_t)(l % 32);
   const uint4* const sbase = reinterpret_cast<const uint4*>(Xs);
-  const uint32_t soff = (uint32_t)l * 2u;
   const int nj = 2 * own_groups<NW>(npad, w);  // this wave's 32-row blocks
   // block of step j; past the end the wave's last block again (read only, unused)
   auto blk_of = [&](int j) {
@@ -498,43 +550,47 @@ __device__ __forceinline__ void field_pass(Smem<NW>& S, const float* __restrict_
   };
   auto fetch_xf = [&](XF& f, int rb) {
     const uint4* const blk = sbase + (size_t)rb * (KC * 128);
+    const uint32_t o = here(xo);
 #pragma unroll
     for (int kc = 0; kc < KC; ++kc) {
-      const uint32_t i = (uint32_t)kc * 128u + soff;
-      f.xh[kc] = __builtin_bit_cast(bf16x8, blk[i]);
-      f.xl[kc] = __builtin_bit_cast(bf16x8, blk[i + 1u]);
+      const uint4* const p = at_byte(blk + kc * 128, o);
+      f.xh[kc] = __builtin_bit_cast(bf16x8, p[0]);
+      f.xl[kc] = __builtin_bit_cast(bf16x8, p[1]);
     }
   };
   auto fetch_blk = [&](Blk& B, int rb) {
     const float* const blk = Xr + (size_t)rb * (KC * 512);
+    const uint32_t o = here(xo), r = here(ro);
 #pragma unroll
-    for (int kc = 0; kc < KC; ++kc) load8(blk + ((uint32_t)kc * 512u + xoff), B.x[kc]);
-    const uint32_t lr = (uint32_t)(l % 32);
-    B.eta = (E1 + (size_t)rb * 32)[lr];
-    B.base = (E0 + (size_t)rb * 32)[lr];  // unused by the explicit step (no branch in the loop)
-    B.yv = (yf + (size_t)rb * 32)[lr];
+    for (int kc = 0; kc < KC; ++kc) load8(at_byte(blk + kc * 512, o), B.x[kc]);
+    B.eta = *at_byte(E1 + rb * 32, r);
+    B.base = *at_byte(E0 + rb * 32, r);  // unused by the explicit step (no branch in the loop)
+    B.yv = *at_byte(yf + rb * 32, r);
   };
-  // The split G^-1 fragments of step tk + 1 are read from LDS while the three
-  // MFMAs of step tk run (one step ahead: two fragments in flight).
-  auto mfma_blk = [&](const XF& f, Blk& B) {
+  // The split G^-1 fragments of product f + 1 are read from LDS while the three
+  // MFMAs of product f run (one step ahead: two fragments in flight).
+  auto mfma_blk = [&](const XF& x, Blk& B) {
     bf16x8 ah = AH[l], al = AL[l];
+    int f = 0;
 #pragma unroll
-    for (int tk = 0; tk < NTK; ++tk) {
-      const int tt = tk / KC, kc = tk % KC;
-      bf16x8 nh = ah, nl = al;
-      if (tk + 1 < NTK) {
-        nh = AH[(tk + 1) * 64 + l];
-        nl = AL[(tk + 1) * 64 + l];
+    for (int kc = 0; kc < KC; ++kc)
+#pragma unroll
+      for (int tt = kc / 2; tt < NB; ++tt) {
+        bf16x8 nh = ah, nl = al;
+        if (f + 1 < NF) {
+          nh = AH[(f + 1) * 64 + l];
+          nl = AL[(f + 1) * 64 + l];
+        }
+        if (kc == 0) B.acc[tt] = f32x16{0};
+        B.acc[tt] = mfma3(ah, al, x.xh[kc], x.xl[kc], B.acc[tt]);
+        if (f + 1 < NF) {
+          __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);  // the next product's two LDS reads
+          __builtin_amdgcn_sched_group_barrier(0x008, 3, 0);  // then this product's three MFMAs
+        }
+        ah = nh;
+        al = nl;
+        ++f;
       }
-      if (kc == 0) B.acc[tt] = f32x16{0};
-      B.acc[tt] = mfma3(ah, al, f.xh[kc], f.xl[kc], B.acc[tt]);
-      if (tk + 1 < NTK) {
-        __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);  // the next step's two LDS reads
-        __builtin_amdgcn_sched_group_barrier(0x008, 3, 0);  // then this step's three MFMAs
-      }
-      ah = nh;
-      al = nl;
-    }
   };
   auto bdot = [&](Blk& B) {
     float bp = 0.0f;
@@ -549,7 +605,6 @@ __device__ __forceinline__ void field_pass(Smem<NW>& S, const float* __restrict_
   };
   float* const e0_dst = explicit_step ? E0 : E1;
   auto post = [&](const Blk& B, int rb) {
-    const int row = rb * 32 + (l % 32);
     float ap = 0.0f;
 #pragma unroll
     for (int tt = 0; tt < NB; ++tt)
@@ -568,17 +623,19 @@ __device__ __forceinline__ void field_pass(Smem<NW>& S, const float* __restrict_
       for (int i = 0; i < 8; ++i) dacc[kc][i] = fmaf(hv, B.x[kc][i], dacc[kc][i]);
     const float en = fmaf(hs, B.b, explicit_step ? B.eta : B.base);
     const float sn = sigmoidf(en);
-    E1[row] = en;
-    e0_dst[row] = en;  // E1 again for a fixed-point iterate (no branch in the loop)
-    SL[row] = sqrt_fast(sn * (1.0f - sn));
+    const uint32_t r = here(ro);
+    *at_byte(E1 + rb * 32, r) = en;
+    *at_byte(e0_dst + rb * 32, r) = en;  // E1 again for a fixed-point iterate (no branch in the loop)
+    *at_byte(SL + rb * 32, r) = sqrt_fast(sn * (1.0f - sn));
   };
   XF f;
   Blk B;
   fetch_xf(f, blk_of(0));
+  __builtin_amdgcn_sched_barrier(0);  // the loop's order of loads (as in gram_pass)
   fetch_blk(B, blk_of(0));
   for (int j = 0; j < nj; ++j) {
     // the A operand is read from LDS per block: holding it in registers
-    // across the loop would cost 64 of them
+    // across the loop would cost 48 of them
     asm volatile("" ::: "memory");
     const int rb = blk_of(j);
     mfma_blk(f, B);
@@ -605,7 +662,7 @@ template <int NB, int NW>
 __device__ __forceinline__ double fresh_pass(Smem<NW>& S, const float* __restrict__ Xr, const float* __restrict__ yf, int N, int npad,
                              int D, float* Eout, float* SL, bool want_grad, float inv_prior) {
   constexpr int KC = 2 * NB;
-  const int t = threadIdx.x, l = t % 64, w = wave_id(), h = l / 32;
+  const int l = pass_lane(), w = wave_id(), t = 64 * w + l, h = l / 32;
   double qv[KC][8];
   float gacc[KC][8];
 #pragma unroll
@@ -616,13 +673,13 @@ __device__ __forceinline__ double fresh_pass(Smem<NW>& S, const float* __restric
       gacc[kc][i] = 0.0f;
     }
   double ll = 0.0;
-  const float* xp = Xr + (size_t)l * 8;
+  const uint32_t xo = 32u * (uint32_t)l;
   const int nj = 2 * own_groups<NW>(npad, w);  // this wave's 32-row blocks
   for (int j = 0; j < nj; ++j) {
     const int rb = own_block<NW>(j, w);
     float x[KC][8];
 #pragma unroll
-    for (int kc = 0; kc < KC; ++kc) load8(xp + (size_t)(rb * KC + kc) * 512, x[kc]);
+    for (int kc = 0; kc < KC; ++kc) load8(at_byte(Xr + (size_t)(rb * KC + kc) * 512, here(xo)), x[kc]);
     double ep = 0.0;
 #pragma unroll
     for (int kc = 0; kc < KC; ++kc)
@@ -657,7 +714,7 @@ __device__ __forceinline__ double fresh_pass(Smem<NW>& S, const float* __restric
 // E0 = E1 = ES, SL = sqrt(lambda(ES))
 template <int NW>
 __device__ __forceinline__ void prep_pass(const float* ES, float* E0, float* E1, float* SL, int npad) {
-  const int l = threadIdx.x % 64, w = wave_id();
+  const int l = pass_lane(), w = wave_id();
   const int ng = own_groups<NW>(npad, w);
   for (int g = 0; g < ng; ++g) {
     const int row = 64 * (w + NW * g) + l;
@@ -679,7 +736,7 @@ __device__ __forceinline__ void lmc_row_pass(Smem<1>& S, const float* __restrict
                                              float* SS, int npad, int D, float coef, float eps, bool want_gv,
                                              bool step, float inv_prior) {
   constexpr int KC = 2 * NB;
-  const int l = threadIdx.x % 64, h = l / 32;
+  const int l = pass_lane(), h = l / 32;
   float v[KC][8], gacc[KC][8];
 #pragma unroll
   for (int kc = 0; kc < KC; ++kc) {
@@ -687,11 +744,11 @@ __device__ __forceinline__ void lmc_row_pass(Smem<1>& S, const float* __restrict
 #pragma unroll
     for (int i = 0; i < 8; ++i) gacc[kc][i] = 0.0f;
   }
-  const float* xp = Xr + (size_t)l * 8;
+  const uint32_t xo = 32u * (uint32_t)l;
   const int nj = npad / 32;  // even: npad is a multiple of 64
   auto fetch = [&](float (&x)[KC][8], float& eta, int rb) {
 #pragma unroll
-    for (int kc = 0; kc < KC; ++kc) load8(xp + (size_t)(rb * KC + kc) * 512, x[kc]);
+    for (int kc = 0; kc < KC; ++kc) load8(at_byte(Xr + (size_t)(rb * KC + kc) * 512, here(xo)), x[kc]);
     eta = ETA[rb * 32 + (l % 32)];
   };
   auto block = [&](const float (&x)[KC][8], float eta, int rb) {

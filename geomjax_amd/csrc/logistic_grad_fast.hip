@@ -118,27 +118,41 @@ __device__ __forceinline__ void tangent_field_pass(TSmem& S, const float* __rest
                                                    const float* __restrict__ Xs, const float* __restrict__ yf,
                                                    float* E0, float* E1, float* TE0, float* TE1, int npad, int D,
                                                    float hs, float inv_prior, bool explicit_step) {
-  constexpr int KC = 2 * NB, NTK = NB * KC;
-  const int l = threadIdx.x % 64, h = l / 32;
+  // products of the lower 32-feature tiles only, the off-diagonal ones doubled, for
+  // both matrices (lfast::field_pass)
+  constexpr int KC = 2 * NB, NF = NB * (NB + 1);
+  const int l = pass_lane(), h = l / 32;
   bf16x8* const AH = reinterpret_cast<bf16x8*>(S.G);
-  bf16x8* const AL = AH + NTK * 64;
+  bf16x8* const AL = AH + NF * 64;
   bf16x8* const TH = reinterpret_cast<bf16x8*>(S.GT);
-  bf16x8* const TL = TH + NTK * 64;
-  static_assert(2 * NTK * 64 * sizeof(bf16x8) <= sizeof(S.GT), "the split operands must fit");
+  bf16x8* const TL = TH + NF * 64;
+  static_assert(2 * NF * 64 * sizeof(bf16x8) <= sizeof(S.GT), "the split operands must fit");
   // stage the split A operands (rows permuted by phi, as the field pass) over
   // the matrices they come from: every read of a matrix before its writes
   auto stage = [&](float* M, bf16x8* H, bf16x8* Lo) {
-    float v[NTK][8];
+    float v[NF][8];
+    int f = 0;
 #pragma unroll
-    for (int tk = 0; tk < NTK; ++tk) load8(M + phi((tk / KC) * 32 + (l % 32)) * LDG + (tk % KC) * 16 + h * 8, v[tk]);
+    for (int kc = 0; kc < KC; ++kc)
+#pragma unroll
+      for (int tt = kc / 2; tt < NB; ++tt) {
+        load8(M + phi(tt * 32 + (l % 32)) * LDG + kc * 16 + h * 8, v[f]);
+        ++f;
+      }
     __syncthreads();
+    f = 0;
 #pragma unroll
-    for (int tk = 0; tk < NTK; ++tk) {
-      bf16x8 hi, lo;
-      split8(v[tk], hi, lo);
-      H[tk * 64 + l] = hi;
-      Lo[tk * 64 + l] = lo;
-    }
+    for (int kc = 0; kc < KC; ++kc)
+#pragma unroll
+      for (int tt = kc / 2; tt < NB; ++tt) {
+#pragma unroll
+        for (int i = 0; i < 8; ++i) v[f][i] *= tt > kc / 2 ? 2.0f : 1.0f;
+        bf16x8 hi, lo;
+        split8(v[f], hi, lo);
+        H[f * 64 + l] = hi;
+        Lo[f * 64 + l] = lo;
+        ++f;
+      }
   };
   stage(S.G, AH, AL);
   stage(S.GT, TH, TL);
@@ -153,33 +167,62 @@ __device__ __forceinline__ void tangent_field_pass(TSmem& S, const float* __rest
     }
   const uint4* const sbase = reinterpret_cast<const uint4*>(Xs);
   const int nj = npad / 32;
+  const uint32_t xo = 32u * (uint32_t)l, ro = 4u * (uint32_t)(l % 32);
+  // Loads run ahead of their use into the registers that their predecessors
+  // leave: the MFMA operands of the next block once this block's products are
+  // issued (the VALU work covers them), its rows and row scalars at the block's end
+  // (the next products cover them).
+  float x[KC][8];
+  bf16x8 xh[KC], xl[KC];
+  float eta, teta, yv, e0, te0;
+  float* const e0_dst = explicit_step ? E0 : E1;  // E1 again for a fixed-point iterate (no branch in the loop)
+  float* const te0_dst = explicit_step ? TE0 : TE1;
+  auto fetch_xf = [&](int rb) {
+    const uint4* const sblk = sbase + (size_t)rb * (KC * 128);
+    const uint32_t o = here(xo);
+#pragma unroll
+    for (int kc = 0; kc < KC; ++kc) {
+      const uint4* const p = at_byte(sblk + kc * 128, o);
+      xh[kc] = __builtin_bit_cast(bf16x8, p[0]);
+      xl[kc] = __builtin_bit_cast(bf16x8, p[1]);
+    }
+  };
+  auto fetch_x = [&](int rb) {
+    const float* const blk = Xr + (size_t)rb * (KC * 512);
+    const uint32_t o = here(xo), r = here(ro);
+#pragma unroll
+    for (int kc = 0; kc < KC; ++kc) load8(at_byte(blk + kc * 512, o), x[kc]);
+    eta = *at_byte(E1 + rb * 32, r);
+    teta = *at_byte(TE1 + rb * 32, r);
+    yv = *at_byte(yf + rb * 32, r);
+    e0 = *at_byte(E0 + rb * 32, r);
+    te0 = *at_byte(TE0 + rb * 32, r);
+  };
+  if (nj > 0) {
+    fetch_xf(0);
+    __builtin_amdgcn_sched_barrier(0);
+    fetch_x(0);
+  }
   for (int rb = 0; rb < nj; ++rb) {
-    float x[KC][8];
-    bf16x8 xh[KC], xl[KC];
-    {
-      const float* const blk = Xr + (size_t)rb * (KC * 512);
-      const uint4* const sblk = sbase + (size_t)rb * (KC * 128);
-      // the MFMA operands first (the first product waits only for its own),
-      // then the rows of X, first read after the products are issued
-#pragma unroll
-      for (int kc = 0; kc < KC; ++kc) {
-        xh[kc] = __builtin_bit_cast(bf16x8, sblk[kc * 128 + l * 2]);
-        xl[kc] = __builtin_bit_cast(bf16x8, sblk[kc * 128 + l * 2 + 1]);
-      }
-#pragma unroll
-      for (int kc = 0; kc < KC; ++kc) load8(blk + kc * 512 + l * 8, x[kc]);
-    }
+    asm volatile("" ::: "memory");  // the staged operands are read from LDS per block
+    const int next = rb + 1 < nj ? rb + 1 : rb;  // past the end the last block again (in bounds, unused)
     f32x16 acc[NB], tac[NB];
+    {
+      int f = 0;
 #pragma unroll
-    for (int tk = 0; tk < NTK; ++tk) {
-      const int tt = tk / KC, kc = tk % KC;
-      if (kc == 0) {
-        acc[tt] = f32x16{0};
-        tac[tt] = f32x16{0};
-      }
-      acc[tt] = mfma3(AH[tk * 64 + l], AL[tk * 64 + l], xh[kc], xl[kc], acc[tt]);
-      tac[tt] = mfma3(TH[tk * 64 + l], TL[tk * 64 + l], xh[kc], xl[kc], tac[tt]);
+      for (int kc = 0; kc < KC; ++kc)
+#pragma unroll
+        for (int tt = kc / 2; tt < NB; ++tt) {
+          if (kc == 0) {
+            acc[tt] = f32x16{0};
+            tac[tt] = f32x16{0};
+          }
+          acc[tt] = mfma3(AH[f * 64 + l], AL[f * 64 + l], xh[kc], xl[kc], acc[tt]);
+          tac[tt] = mfma3(TH[f * 64 + l], TL[f * 64 + l], xh[kc], xl[kc], tac[tt]);
+          ++f;
+        }
     }
+    fetch_xf(next);
     float bp = 0.0f, tbp = 0.0f;
 #pragma unroll
     for (int kc = 0; kc < KC; ++kc) {
@@ -203,8 +246,6 @@ __device__ __forceinline__ void tangent_field_pass(TSmem& S, const float* __rest
         tap = fmaf(tac[tt][r], x[j / 8][j % 8], tap);
       }
     const float an = ap + __shfl_xor(ap, 32, 64), tan_ = tap + __shfl_xor(tap, 32, 64);
-    const int row = rb * 32 + (l % 32);
-    const float eta = E1[row], teta = TE1[row], yv = yf[row];
     const float s = sigmoidf(eta);
     const float lam = s * (1.0f - s);
     const float wv = lam * (1.0f - 2.0f * s);
@@ -220,18 +261,17 @@ __device__ __forceinline__ void tangent_field_pass(TSmem& S, const float* __rest
         dacc[kc][i] = fmaf(hv, x[kc][i], dacc[kc][i]);
         tacc[kc][i] = fmaf(thv, x[kc][i], tacc[kc][i]);
       }
-    const float base = explicit_step ? eta : E0[row];
-    const float tbase = explicit_step ? teta : TE0[row];
+    const float base = explicit_step ? eta : e0;
+    const float tbase = explicit_step ? teta : te0;
     const float en = fmaf(hs, b, base);
     const float ten = fmaf(hs, b + tb, tbase);  // d(hs)/d log eps = hs
-    if (h == 0) {
-      E1[row] = en;
-      TE1[row] = ten;
-      if (explicit_step) {
-        E0[row] = en;
-        TE0[row] = ten;
-      }
-    }
+    const uint32_t r = here(ro);
+    *at_byte(E1 + rb * 32, r) = en;
+    *at_byte(TE1 + rb * 32, r) = ten;
+    *at_byte(e0_dst + rb * 32, r) = en;
+    *at_byte(te0_dst + rb * 32, r) = ten;
+    __builtin_amdgcn_sched_barrier(0);
+    fetch_x(next);
   }
   const float tot = reduce_features<NB, 1>(S, dacc);
   S.dH[l] = l < D ? tot + S.q[l] * inv_prior : 0.0f;
