@@ -40,6 +40,30 @@ __device__ __forceinline__ FieldCoef<R> field_coef(R v, R pv, R sx, R xpx, R a2,
   return f;
 }
 
+// Whether the fixed-point iteration goes on, decided without the per-coordinate
+// norm where that is certain.  The norm is the largest of |da x0_k + db p0_k| and
+// |dg x0_k + dd p0_k| over the coordinates and of mv, the change of v and p_v.
+// With |x0_k| <= X and |p0_k| <= P (2-norms, with slack for their rounding)
+//   norm >= mv  and  norm <= max(|da| X + |db| P, |dg| X + |dd| P, mv),
+// so mv > tol with the upper bound below the divergence limit goes on, an upper
+// bound within tol has converged, and a non-finite change (norm NaN) stops.
+// Everything else is kOpen: the norm itself has to be formed.  Comparisons with
+// NaN are false, which leads there.
+enum SpanDecision { kStop, kGoOn, kOpen };
+
+struct SpanBound {
+  float X, P;
+  __device__ __forceinline__ SpanBound(float Sxx, float Spp) : X(1.001f * sqrtf(Sxx)), P(1.001f * sqrtf(Spp)) {}
+  __device__ __forceinline__ SpanDecision operator()(bool finite, float mv, float da, float db, float dg, float dd,
+                                                     double tol, double div_tol) const {
+    const float up = 1.001f * fmaxf(fmaxf(fabsf(da) * X + fabsf(db) * P, fabsf(dg) * X + fabsf(dd) * P), mv);
+    if (!finite || mv != mv) return kStop;
+    if ((double)mv > tol && (double)up < div_tol) return kGoOn;
+    if ((double)up <= tol) return kStop;
+    return kOpen;
+  }
+};
+
 // Quadratic form p^T G^-1 p of the Monge metric G = I + a2 g g^T, written as
 //   |p|^2 / L + (a2 |g|^2 / L) |p_perp|^2,   L = 1 + a2 |g|^2,
 //   p_perp = p - (g.p / |g|^2) g   (formed component by component).

@@ -413,26 +413,33 @@ __global__ void __launch_bounds__(64) funnel_nuts_kernel(const FunnelArgs a, con
     int n = -1;
     double norm = 0.0;
     if constexpr (sizeof(T) == sizeof(float)) {
-      // the iterates in span{x0, p0} (funnel_rmhmc.hip): x = ca x0 + cb p0, p = cg x0 + cd p0
+      // the iterates in span{x0, p0} (funnel_rmhmc.hip): x = ca x0 + cb p0, p = cg x0 + cd p0,
+      // the norm formed only where its bounds leave the decision open
       T spp = T(0);
 #pragma unroll
       for (int k = 0; k < EPL; ++k) spp += p0[k] * p0[k];
       const T Sxx = s.sx, Sxp = s.xpx, Spp = group_sum<64>(spp);
+      const SpanBound bound((float)Sxx, (float)Spp);
       T ca = T(1), cb = T(0), cg = T(0), cd = T(1);
       while (true) {
         const FieldCoef<T> f = field_coef<T>(s.v, s.pv, s.sx, s.xpx, a2, inv_s2, halfDx);
         const T na = T(1) + h * (cg + f.ce * ca), nb = h * (cd + f.ce * cb);
         const T ng = -h * (f.A * ca + f.B * cg), nd = T(1) - h * (f.A * cb + f.B * cd);
         const T da = na - ca, db = nb - cb, dg = ng - cg, dd = nd - cd;
-        T mx = T(0);
-#pragma unroll
-        for (int k = 0; k < EPL; ++k)
-          mx = fmaxf(mx, fmaxf(fabsf(da * x0[k] + db * p0[k]), fabsf(dg * x0[k] + dd * p0[k])));
-        mx = group_reduce<64, OpMax>(mx);
         const T vn = v0 + h * f.uv;
         const T pvn = pv0 - h * f.dHv;
-        mx = nan_max(mx, nan_max(fabsf(vn - s.v), fabsf(pvn - s.pv)));
-        if (!isfinite(na + nb + ng + nd)) mx = T(NAN);
+        const T mv = nan_max(fabsf(vn - s.v), fabsf(pvn - s.pv));
+        const bool finite = isfinite(na + nb + ng + nd);
+        ++n;
+        SpanDecision dec = n < a.max_iters ? bound(finite, mv, da, db, dg, dd, a.conv_tol, a.div_tol) : kStop;
+        if (dec == kOpen) {
+          T mx = T(0);
+#pragma unroll
+          for (int k = 0; k < EPL; ++k)
+            mx = fmaxf(mx, fmaxf(fabsf(da * x0[k] + db * p0[k]), fabsf(dg * x0[k] + dd * p0[k])));
+          mx = nan_max(group_reduce<64, OpMax>(mx), mv);
+          dec = isfinite(mx) && (double)mx < a.div_tol && (double)mx > a.conv_tol ? kGoOn : kStop;
+        }
         ca = na;
         cb = nb;
         cg = ng;
@@ -441,9 +448,7 @@ __global__ void __launch_bounds__(64) funnel_nuts_kernel(const FunnelArgs a, con
         s.pv = pvn;
         s.sx = (ca * ca) * Sxx + (T(2) * ca * cb) * Sxp + (cb * cb) * Spp;
         s.xpx = (ca * cg) * Sxx + (ca * cd + cb * cg) * Sxp + (cb * cd) * Spp;
-        norm = (double)mx;
-        ++n;
-        if (!(n < a.max_iters && isfinite(norm) && norm < a.div_tol && norm > a.conv_tol)) break;
+        if (dec == kStop) break;
       }
 #pragma unroll
       for (int k = 0; k < EPL; ++k) {
