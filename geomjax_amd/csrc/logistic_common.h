@@ -29,6 +29,16 @@
 namespace gjx {
 namespace logistic {
 
+// The lane's index in the workgroup, opaque to the compiler: addresses formed from it
+// inside a pass are not hoisted above the stage loop of a chain, where they only spill.
+// At capacity 64 the RMHMC loop spilled 157 registers without it and 84 with it (2048 x 64,
+// 1024 chains: 30.7 -> 30.3 ms), MMALA 159 and 86 (four transitions: 5.68 -> 5.46 ms).
+__device__ __forceinline__ int pass_thread() {
+  int t = (int)threadIdx.x;
+  asm volatile("" : "+v"(t));
+  return t;
+}
+
 constexpr int NT = 256;
 
 template <int MD>
@@ -148,7 +158,7 @@ __device__ __forceinline__ void gram_loop(Smem<C>& S, const double* X, const dou
                                           double coef, bool want_gv, int w, f64x4 (&acc)[NTW], double& ll,
                                           double (&gacc)[NB], double (&gvacc)[NB]) {
   constexpr int WR = 4 / C::H;
-  const int l = threadIdx.x % 64;
+  const int l = pass_thread() % 64;
   const int g = l / 16, m = l % 16;
   const int nblk = (N + 15) / 16;
   if (nblk == 0) return;
@@ -271,7 +281,7 @@ template <class C, int NB, bool VEC, bool LG>
 __device__ __forceinline__ void gram_pass_nb(Smem<C>& S, const double* X, const double* y, int N, int D, double prior_var,
                                              const double* vec, double coef, bool want_gv, double& loglik) {
   constexpr int NTL = NB * (NB + 1) / 2, NTW = (NTL + C::H - 1) / C::H;
-  const int t = threadIdx.x, l = t % 64, w = __builtin_amdgcn_readfirstlane(t / 64);
+  const int t = pass_thread(), l = t % 64, w = __builtin_amdgcn_readfirstlane((int)threadIdx.x / 64);
   f64x4 acc[NTW];
 #pragma unroll
   for (int i = 0; i < NTW; ++i) acc[i] = f64x4{0, 0, 0, 0};
@@ -405,7 +415,7 @@ __device__ __forceinline__ void pass1(Smem<C>& S, const double* X, const double*
 // Load this lane's BS x BS block of S.Gi into registers (entries past D are 0).
 template <class C>
 __device__ __forceinline__ void load_block(const Smem<C>& S, double (&A)[C::BS][C::BS], int D) {
-  const int t = threadIdx.x;
+  const int t = pass_thread();
   const int i0 = C::BS * (t / 16), j0 = C::BS * (t % 16);
 #pragma unroll
   for (int a = 0; a < C::BS; ++a)
@@ -430,7 +440,7 @@ template <class C>
 __device__ __forceinline__ void sweep(Smem<C>& S, double (&A)[C::BS][C::BS], int D, const double* zc = nullptr,
                                       double* pout = nullptr) {
   constexpr int BS = C::BS;
-  const int t = threadIdx.x;
+  const int t = pass_thread();
   const int i0 = BS * (t / 16), j0 = BS * (t % 16);
   double pacc = 0.0;
   for (int kk = 0; kk * BS < D; ++kk) {
@@ -473,14 +483,14 @@ __device__ __forceinline__ void sweep(Smem<C>& S, double (&A)[C::BS][C::BS], int
 template <class C>
 __device__ __forceinline__ double pivots_logdet(Smem<C>& S, int D) {
   __syncthreads();  // the last pivot's write
-  const int t = threadIdx.x;
+  const int t = pass_thread();
   return block_sum(S, t < D ? log(fabs(S.dk[t])) : 0.0);
 }
 
 // Write G^-1 = -A into S.Gi.
 template <class C>
 __device__ __forceinline__ void store_neg_block(Smem<C>& S, const double (&A)[C::BS][C::BS]) {
-  const int t = threadIdx.x;
+  const int t = pass_thread();
   const int i0 = C::BS * (t / 16), j0 = C::BS * (t % 16);
 #pragma unroll
   for (int a = 0; a < C::BS; ++a)
@@ -493,7 +503,7 @@ __device__ __forceinline__ void store_neg_block(Smem<C>& S, const double (&A)[C:
 // columns: one barrier per pivot.  Returns log det (= 2 sum log L_kk).
 template <class C>
 __device__ double cholesky(Smem<C>& S, int D) {
-  const int t = threadIdx.x, w = t / 64, l = t % 64;
+  const int t = pass_thread(), w = t / 64, l = t % 64;
   for (int k = 0; k < D; ++k) {
     const double rd = 1.0 / S.Gi[k * C::LDX + k];
     for (int i = k + 1 + w; i < D; i += 4) {
@@ -523,7 +533,7 @@ __device__ double cholesky(Smem<C>& S, int D) {
 template <class C>
 __device__ __forceinline__ void ginv_times(Smem<C>& S, const double* p, double* out, int D) {
   constexpr int TPR = NT / C::MAXD;
-  const int r = threadIdx.x / TPR, h = threadIdx.x % TPR;
+  const int pt = pass_thread(), r = pt / TPR, h = pt % TPR;
   double s = 0.0;
   if (r < D)
     for (int j = h; j < D; j += TPR) s += S.Gi[r * C::LDX + j] * p[j];
@@ -557,7 +567,7 @@ __device__ __forceinline__ void quad_pass_nb(Smem<C>& S, const double* X, const 
                                              double prior_var) {
   constexpr int NS = 4 * NB;
   constexpr bool REG = C::MAXD == 64;
-  const int t = threadIdx.x, l = t % 64, w = __builtin_amdgcn_readfirstlane(t / 64);
+  const int t = pass_thread(), l = t % 64, w = __builtin_amdgcn_readfirstlane((int)threadIdx.x / 64);
   const int g = l / 16, m = l % 16;
   const int nblk = (N + 15) / 16;
   auto feat = [](int s, int gg) { return 8 * (s / 2) + 2 * gg + s % 2; };
