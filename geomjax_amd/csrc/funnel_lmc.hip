@@ -15,8 +15,7 @@
 //   igHdl_x = mi Hdl_x                   (ig_Hdl_ig)
 //   hv_x = e (-vel_x + x vel_v) / sqrt(L)  (logdensity_hvp_velocity_norm)
 // and the dot products half_step_omega needs are linear in the velocity, so
-// four sums with the velocity per half step and four sums per position (funnel_lmc_ops.h)
-// give all of them:
+// one group reduction of eight sums per half step gives all of them:
 //   v_t.hv  = v.hv - (eps/2) sqrt(L) (dphi_ig.hv - alpha2 (dphi.dl) (dl.hv))
 //   Hdl.v'  = Hdl.v - (eps/2) sqrt(L) (Hdl.dphi_ig - alpha2 (dphi.dl)(Hdl.dl)) - c (Hdl.dl).
 // The velocity draw v0 = chol(M^-1 - alpha2 dl dl^T) z uses the exact lower

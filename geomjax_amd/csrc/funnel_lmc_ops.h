@@ -18,34 +18,11 @@ namespace lmc_ops {
 template <class R>
 struct PosScalars {
   R e, Sx, Smx, gv, L, sL, isL, dlv, Hdlv, igHdlv;
-  R eL;          // e / sqrt(L)
-  R Q1, Q2, Q3;  // eL sum mi x^2, eL^2 sum mi^2 x^2, eL^2 sum mi^3 x^2
-};
-
-// Sums over a position's coordinates: x^2, mi x^2, mi^2 x^2, mi^3 x^2.
-template <class R>
-struct PosSums {
-  R x2 = R(0), mx2 = R(0), m2x2 = R(0), m3x2 = R(0);
-  __device__ __forceinline__ void add(R x, R mi) {
-    const R t = mi * x, u = mi * t;
-    x2 += x * x;
-    mx2 += t * x;
-    m2x2 += t * t;
-    m3x2 += u * t;
-  }
-  template <int LPC>
-  __device__ __forceinline__ void reduce() {
-    x2 = group_sum<LPC>(x2);
-    mx2 = group_sum<LPC>(mx2);
-    m2x2 = group_sum<LPC>(m2x2);
-    m3x2 = group_sum<LPC>(m3x2);
-  }
 };
 
 template <class R>
-__device__ __forceinline__ PosScalars<R> pos_scalars(R v, const PosSums<R>& S, R a2, R inv_s2, R halfDx, R miv) {
+__device__ __forceinline__ PosScalars<R> pos_scalars(R v, R Sx, R Smx, R a2, R inv_s2, R halfDx, R miv) {
   PosScalars<R> P;
-  const R Sx = S.x2, Smx = S.mx2;
   P.e = exp(-v);
   P.Sx = Sx;
   P.Smx = Smx;
@@ -57,57 +34,44 @@ __device__ __forceinline__ PosScalars<R> pos_scalars(R v, const PosSums<R>& S, R
   // Hdl_v = (e (x . dl_x) - (1/sigma^2 + e Sx / 2) dl_v) / sqrt(L),  x . dl_x = -e Smx / sqrt(L)
   P.Hdlv = (-P.e * P.e * Smx * P.isL - (inv_s2 + R(0.5) * P.e * Sx) * P.dlv) * P.isL;
   P.igHdlv = miv * P.Hdlv;
-  // eL meets a sum one factor at a time: its square alone may leave R's range
-  P.eL = P.e * P.isL;
-  P.Q1 = P.eL * Smx;
-  P.Q2 = P.eL * (P.eL * S.m2x2);
-  P.Q3 = P.eL * (P.eL * S.m3x2);
   return P;
 }
 
 // One half_step_omega (geomjax/lmcmonge/integrators.py:158-194) at the
 // position described by P, updating the velocity (vx, vv) and dJ.
-//
-// Every vector of the half step is a combination of x, mi x, mi^2 x and the
-// velocity (t = mi x, u = mi t below), so its dot products s0 .. s7 are
-// combinations of the position's sums Q1 .. Q3, formed once per position for both
-// half steps that meet there, and of four sums with the velocity.  VALU issue and the
-// chain of group sums bound the kernel: a step takes 12 of them (18 with each dot
-// product summed by itself) and about half the instructions per coordinate (8192 chains,
-// 100 float32 coordinates, 4 transitions of 32 steps: 448 -> 368 us; the position's
-// error against float64 arithmetic 6.0e-4 -> 5.3e-4).
-//   dl = -eL t,  Hdl = eL (eL t + dlv x),  hv = eL (vv x - v),
-//   dphi = g0 x + k1 eL^2 t,  dphi_ig = mi dphi,  g0 = eL (1 + k1 dlv), k1 = alpha2 / sqrt(L).
 template <class R, int LPC, int EPL>
 __device__ __forceinline__ void half_step(const PosScalars<R>& P, const R (&x)[EPL], const R (&mi)[EPL], R (&vx)[EPL],
                                           R& vv, double& dJ, R a2, R inv_s2, R h, bool exact_sm) {
-  R xv = R(0), tv = R(0), uv = R(0), v2 = R(0);
+  R dl[EPL], dphig[EPL];
+  R s0 = R(0), s1 = R(0), s2 = R(0), s3 = R(0), s4 = R(0), s5 = R(0), s6 = R(0), s7 = R(0);
 #pragma unroll
   for (int k = 0; k < EPL; ++k) {
-    const R t = mi[k] * x[k], u = mi[k] * t;
-    xv += x[k] * vx[k];
-    tv += t * vx[k];
-    uv += u * vx[k];
-    v2 += vx[k] * vx[k];
+    const R gn = -P.e * x[k] * P.isL;
+    dl[k] = mi[k] * gn;
+    const R Hdl = P.e * (-dl[k] + x[k] * P.dlv) * P.isL;
+    const R igH = mi[k] * Hdl;
+    const R dphi = -gn + a2 * Hdl * P.isL;
+    dphig[k] = -dl[k] + a2 * igH * P.isL;
+    const R hv = P.e * (-vx[k] + x[k] * vv) * P.isL;
+    s0 += hv * dl[k];
+    s1 += dphi * dl[k];
+    s2 += x[k] * vx[k];
+    s3 += vx[k] * hv;
+    s4 += dphig[k] * hv;
+    s5 += Hdl * vx[k];
+    s6 += Hdl * dphig[k];
+    s7 += Hdl * dl[k];
   }
-  xv = group_sum<LPC>(xv);
-  tv = group_sum<LPC>(tv);
-  uv = group_sum<LPC>(uv);
-  v2 = group_sum<LPC>(v2);
-  const R eL = P.eL, k1 = a2 * P.isL, ke = k1 * eL;
-  const R g0 = eL * (R(1) + k1 * P.dlv);
-  const R m1 = eL * tv, m2 = eL * (eL * uv);
-  const R w1 = vv * P.Q1 - m1, w2 = vv * P.Q2 - m2;  // eL sum t (vv x - v), eL^2 sum u (vv x - v)
-  const R q2 = P.Q2 + P.dlv * P.Q1;
-  const R s0 = -eL * w1;                                                    // hv . dl
-  const R s1 = -(g0 * P.Q1 + ke * P.Q2);                                    // dphi . dl
-  const R s3 = eL * (vv * xv - v2);                                         // v . hv
-  const R s4 = g0 * w1 + ke * w2;                                           // dphi_ig . hv
-  const R s5 = eL * (m1 + P.dlv * xv);                                      // Hdl . v
-  const R s6 = g0 * q2 + ke * (eL * P.Q3 + P.dlv * P.Q2);                   // Hdl . dphi_ig
-  const R s7 = -eL * q2;                                                    // Hdl . dl
+  s0 = group_sum<LPC>(s0);
+  s1 = group_sum<LPC>(s1);
+  s2 = group_sum<LPC>(s2);
+  s3 = group_sum<LPC>(s3);
+  s4 = group_sum<LPC>(s4);
+  s5 = group_sum<LPC>(s5);
+  s6 = group_sum<LPC>(s6);
+  s7 = group_sum<LPC>(s7);
   // log-scale coordinate contributions
-  const R hv_v = (P.e * xv - (inv_s2 + R(0.5) * P.e * P.Sx) * vv) * P.isL;
+  const R hv_v = (P.e * s2 - (inv_s2 + R(0.5) * P.e * P.Sx) * vv) * P.isL;
   const R gn_v = P.gv * P.isL;
   const R dphi_v = -gn_v + a2 * P.Hdlv * P.isL;
   const R dphig_v = -P.dlv + a2 * P.igHdlv * P.isL;
@@ -129,12 +93,8 @@ __device__ __forceinline__ void half_step(const PosScalars<R>& P, const R (&x)[E
   // 2nd volume adjustment (:192)
   dJ += log(fabs((double)val(R(1) - h * a2 * HdlVn)));
   const R kq = h * P.sL, kd = a2 * P2;
-  const R ct = eL * (coef - kq * kd) - kq * g0, cu = kq * ke;
 #pragma unroll
-  for (int k = 0; k < EPL; ++k) {
-    const R t = mi[k] * x[k], u = mi[k] * t;
-    vx[k] = vx[k] + ct * t - cu * (eL * u);
-  }
+  for (int k = 0; k < EPL; ++k) vx[k] = vx[k] - kq * (dphig[k] - kd * dl[k]) - coef * dl[k];
   vv = vv - kq * (dphig_v - kd * P.dlv) - coef * P.dlv;
 }
 
@@ -143,17 +103,19 @@ __device__ __forceinline__ void half_step(const PosScalars<R>& P, const R (&x)[E
 template <class R, int LPC, int EPL>
 __device__ __forceinline__ PosScalars<R> position_scalars(const R (&x)[EPL], R v, const R (&mi)[EPL], R (&loc_inc)[EPL],
                                                           int lg, R a2, R inv_s2, R halfDx, R miv) {
-  PosSums<R> S;
+  R sx = R(0), smx = R(0);
 #pragma unroll
   for (int k = 0; k < EPL; ++k) {
-    S.add(x[k], mi[k]);
-    loc_inc[k] = S.mx2;
+    sx += x[k] * x[k];
+    smx += mi[k] * x[k] * x[k];
+    loc_inc[k] = smx;
   }
-  const R off = group_exclusive_scan<LPC>(S.mx2, lg);
+  const R off = group_exclusive_scan<LPC>(smx, lg);
 #pragma unroll
   for (int k = 0; k < EPL; ++k) loc_inc[k] += off;
-  S.template reduce<LPC>();
-  return pos_scalars<R>(v, S, a2, inv_s2, halfDx, miv);
+  sx = group_sum<LPC>(sx);
+  smx = group_sum<LPC>(smx);
+  return pos_scalars<R>(v, sx, smx, a2, inv_s2, halfDx, miv);
 }
 
 // The transition's standard normals for the velocity draw and its accept
@@ -234,15 +196,17 @@ __device__ __forceinline__ void lmc_step(PosScalars<R>& P, R (&xc)[EPL], R& vc, 
                                          R& vv, double& dJ, R eps, R h, R a2, R inv_s2, R halfDx, R miv,
                                          bool exact_sm) {
   half_step<R, LPC, EPL>(P, xc, mi, vx, vv, dJ, a2, inv_s2, h, exact_sm);
-  PosSums<R> S;
+  R sx = R(0), smx = R(0);
 #pragma unroll
   for (int k = 0; k < EPL; ++k) {
     xc[k] = xc[k] + eps * vx[k];
-    S.add(xc[k], mi[k]);
+    sx += xc[k] * xc[k];
+    smx += mi[k] * xc[k] * xc[k];
   }
   vc = vc + eps * vv;
-  S.template reduce<LPC>();
-  P = pos_scalars<R>(vc, S, a2, inv_s2, halfDx, miv);
+  sx = group_sum<LPC>(sx);
+  smx = group_sum<LPC>(smx);
+  P = pos_scalars<R>(vc, sx, smx, a2, inv_s2, halfDx, miv);
   half_step<R, LPC, EPL>(P, xc, mi, vx, vv, dJ, a2, inv_s2, h, exact_sm);
 }
 
