@@ -64,6 +64,18 @@ struct SpanBound {
   }
 };
 
+// Whether a layout of LPC lanes with EPL coordinates each forms the bounds first.  They
+// cost about forty instructions of every iteration's serial chain; the norm they
+// save costs EPL steps and log2(LPC) exchanges, those past a row of 16 lanes through
+// LDS.  Measured against the norm in every iteration, time ratio at 9 | 8192 chains,
+// 18 steps, four transitions (LPC x EPL): 4x1 0.85 | 0.82, 4x4 0.96 | 0.93, 4x8 1.10 | 1.04,
+// 8x4 0.97 | 0.99, 8x8 1.10 | 1.10, 8x16 1.20 | 1.22, 16x1 0.97 | 1.01, 16x2 1.00 | 1.09,
+// 16x8 1.17 | 1.28, 32x1 1.01 | 1.05, 32x4 1.11 | 1.14, 64x1 1.12 | 1.12.
+template <int LPC, int EPL>
+__device__ constexpr bool span_screens() {
+  return EPL >= 8 || LPC >= 32 || (LPC == 16 && EPL >= 2);
+}
+
 // Quadratic form p^T G^-1 p of the Monge metric G = I + a2 g g^T, written as
 //   |p|^2 / L + (a2 |g|^2 / L) |p_perp|^2,   L = 1 + a2 |g|^2,
 //   p_perp = p - (g.p / |g|^2) g   (formed component by component).

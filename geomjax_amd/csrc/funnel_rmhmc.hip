@@ -216,7 +216,8 @@ __global__ void __launch_bounds__(256) funnel_rmhmc_kernel(const FunnelArgs a) {
         //   x = ca x0 + cb p0,  p = cg x0 + cd p0,
         // and |x|^2 and x.p follow from the three sums of the step start.  The
         // convergence norm max |x' - x|, |p' - p| is formed per coordinate only where
-        // its bounds leave the decision open (SpanBound), and in the single-step
+        // its bounds leave the decision open (SpanBound; in every iteration of the layouts
+        // where it is the cheaper of the two, span_screens), and in the single-step
         // form, which returns it, when the iteration stops: it and its group
         // maximum were half of an iteration (8192 chains, D = 100, 32 steps, two
         // transitions: 366 -> 278 us).
@@ -224,6 +225,7 @@ __global__ void __launch_bounds__(256) funnel_rmhmc_kernel(const FunnelArgs a) {
 #pragma unroll
         for (int k = 0; k < EPL; ++k) spp += p0[k] * p0[k];
         const R Sxx = sx, Sxp = xpx, Spp = group_sum<LPC>(spp);
+        constexpr bool kScreen = span_screens<LPC, EPL>();
         const SpanBound bound((float)Sxx, (float)Spp);
         R ca = R(1), cb = R(0), cg = R(0), cd = R(1);
         while (true) {
@@ -232,26 +234,41 @@ __global__ void __launch_bounds__(256) funnel_rmhmc_kernel(const FunnelArgs a) {
           const R na = R(1) + h * (cg + f.ce * ca), nb = h * (cd + f.ce * cb);
           const R ng = -h * (f.A * ca + f.B * cg), nd = R(1) - h * (f.A * cb + f.B * cd);
           const R da = na - ca, db = nb - cb, dg = ng - cg, dd = nd - cd;
-          const R vn = v0 + h * f.uv;
-          const R pvn = pv0 - h * f.dHv;
-          const R mv = nan_max(fabs(vn - vc), fabs(pvn - pvc));
-          const bool finite = isfinite(na + nb + ng + nd);
-          const bool more = n + 1 < a.max_iters;
-          const SpanDecision dec = bound(finite, mv, da, db, dg, dd, a.conv_tol, a.div_tol);
-          bool go = more && dec == kGoOn;
-          if (__any(active && (STEP ? !go : more && dec == kOpen))) {
+          R vn, pvn;
+          bool go = false;
+          if constexpr (kScreen) {
+            vn = v0 + h * f.uv;
+            pvn = pv0 - h * f.dHv;
+            const R mv = nan_max(fabs(vn - vc), fabs(pvn - pvc));
+            const bool finite = isfinite(na + nb + ng + nd);
+            const bool more = n + 1 < a.max_iters;
+            const SpanDecision dec = bound(finite, mv, da, db, dg, dd, a.conv_tol, a.div_tol);
+            go = more && dec == kGoOn;
+            if (__any(active && (STEP ? !go : more && dec == kOpen))) {
+              R mx = R(0);
+#pragma unroll
+              for (int k = 0; k < EPL; ++k)
+                mx = fmaxf(mx, fmaxf(fabsf(da * x0[k] + db * p0[k]), fabsf(dg * x0[k] + dd * p0[k])));
+              mx = group_reduce<LPC, OpMax>(mx);
+              mx = nan_max(mx, mv);
+              // the per-coordinate max drops NaN; a non-finite coefficient (or step
+              // start sum, through the field) makes the norm NaN instead
+              if (!finite) mx = R(NAN);
+              if (active) norm = (double)mx;
+              // cond_fn (integrators.py:67-74)
+              go = more && isfinite(mx) && (double)mx < a.div_tol && (double)mx > a.conv_tol;
+            }
+          } else {
             R mx = R(0);
 #pragma unroll
             for (int k = 0; k < EPL; ++k)
               mx = fmaxf(mx, fmaxf(fabsf(da * x0[k] + db * p0[k]), fabsf(dg * x0[k] + dd * p0[k])));
             mx = group_reduce<LPC, OpMax>(mx);
-            mx = nan_max(mx, mv);
-            // the per-coordinate max drops NaN; a non-finite coefficient (or step
-            // start sum, through the field) makes the norm NaN instead
-            if (!finite) mx = R(NAN);
+            vn = v0 + h * f.uv;
+            pvn = pv0 - h * f.dHv;
+            mx = nan_max(mx, nan_max(fabs(vn - vc), fabs(pvn - pvc)));
+            if (!isfinite(na + nb + ng + nd)) mx = R(NAN);
             if (active) norm = (double)mx;
-            // cond_fn (integrators.py:67-74)
-            go = more && isfinite(mx) && (double)mx < a.div_tol && (double)mx > a.conv_tol;
           }
           if (active) {
             ca = na;
@@ -265,7 +282,10 @@ __global__ void __launch_bounds__(256) funnel_rmhmc_kernel(const FunnelArgs a) {
             ++n;
             ++n_fev;
           }
-          active = active && go;
+          if constexpr (kScreen)
+            active = active && go;
+          else  // cond_fn
+            active = on && n < a.max_iters && isfinite(norm) && norm < a.div_tol && norm > a.conv_tol;
           if (!__any(active)) break;
         }
 #pragma unroll
