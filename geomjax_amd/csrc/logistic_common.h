@@ -25,6 +25,7 @@
 #include <type_traits>
 
 #include "common.h"
+#include "logistic_tiles.h"
 
 namespace gjx {
 namespace logistic {
@@ -124,21 +125,6 @@ __device__ __forceinline__ double sum4_of_16(const double (&e)[4], int l) {
 template <int J>
 __device__ __forceinline__ double quad_bcast(double v) { return dpp<J * 0x55>(v); }
 
-// f(integral_constant<NB>) for the number of 16-feature tiles of a posterior
-// with D features (capacity 128: six or eight tiles).
-template <class C, class F>
-__device__ __forceinline__ void by_width(int D, F f) {
-  if constexpr (C::MAXD == 64) {
-    if (D <= 16) f(std::integral_constant<int, 1>{});
-    else if (D <= 32) f(std::integral_constant<int, 2>{});
-    else if (D <= 48) f(std::integral_constant<int, 3>{});
-    else f(std::integral_constant<int, 4>{});
-  } else {
-    if (D <= 96) f(std::integral_constant<int, 6>{});
-    else f(std::integral_constant<int, 8>{});
-  }
-}
-
 // Gram pass at S.q: S.Gi = X^T diag(lambda + coef w (X vec)) X + I / prior_var
 // (vec == nullptr: the Fisher metric G itself) in the first D rows and columns
 // (nothing meaningful past them: load_block reads zeros there).  With want_lg it
@@ -172,19 +158,19 @@ __device__ __forceinline__ void gram_loop(Smem<C>& S, const double* X, const dou
     double x[4][NB];
     double y;
   };
-  // features past D in the last tile read feature D - 1, rows past N row N - 1
-  // (in bounds; they meet zeros or tile entries that are not used); past its
+  // features past D, all in the last tile, read feature D - 1 and rows past N row
+  // N - 1 (in bounds; they meet zeros or tile entries that are not used); past its
   // last block a wave re-reads the last one with weights of zero
   // (byte offsets from a block's first row: a uniform base, one 32-bit lane offset
   // per K step and immediate offsets per tile)
-  const uint32_t mb = 8u * (uint32_t)m, lastb = 8u * (uint32_t)min(16 * (NB - 1) + m, D - 1);
+  const uint32_t mb = 8u * (uint32_t)m, lastb = last_tile_bytes(NB, m, D);
   uint32_t rowb[4];
 #pragma unroll
   for (int j = 0; j < 4; ++j) rowb[j] = 8u * (uint32_t)((4 * j + g) * D);
   auto fetch_row = [&](Blk& B, int blk, int j) {
     const int n0 = 16 * min(blk, nblk - 1);
     const char* const Xb = reinterpret_cast<const char*>(X + (size_t)n0 * D);
-    const uint32_t row = min(rowb[j], 8u * (uint32_t)(min(N - n0 - 1, 15) * D));
+    const uint32_t row = row_bytes(rowb[j], n0, N, D);
     const double* const xr = reinterpret_cast<const double*>(Xb + (row + mb));
 #pragma unroll
     for (int b = 0; b < NB - 1; ++b) B.x[j][b] = xr[16 * b];
@@ -403,7 +389,7 @@ __device__ __forceinline__ void pass_gram(Smem<C>& S, const double* X, const dou
     else
       gram_pass_nb<C, NB, false, false>(S, X, y, N, D, prior_var, nullptr, 0.0, false, loglik);
   };
-  by_width<C>(D, run);
+  by_width<C::MAXD>(D, run);
 }
 
 template <class C>
@@ -570,31 +556,30 @@ __device__ __forceinline__ void quad_pass_nb(Smem<C>& S, const double* X, const 
   const int t = pass_thread(), l = t % 64, w = __builtin_amdgcn_readfirstlane((int)threadIdx.x / 64);
   const int g = l / 16, m = l % 16;
   const int nblk = (N + 15) / 16;
-  auto feat = [](int s, int gg) { return 8 * (s / 2) + 2 * gg + s % 2; };
   // G^-1[feature of row m of tile tt][F(s, g)], s < 4 (tt + 1), read as the transposed element
-  const int rf = feat(m / 4, m % 4);
+  const int rf = quad_feature(m / 4, m % 4);
   double T[REG ? 2 * NB * (NB + 1) : 1];
   if constexpr (REG) {
     int i = 0;
 #pragma unroll
     for (int tt = 0; tt < NB; ++tt)
 #pragma unroll
-      for (int s = 0; s < 4 * (tt + 1); ++s) T[i++] = S.Gi[feat(s, g) * C::LDX + 16 * tt + rf];
+      for (int s = 0; s < 4 * (tt + 1); ++s) T[i++] = S.Gi[quad_feature(s, g) * C::LDX + 16 * tt + rf];
   }
   double dacc[NS];
 #pragma unroll
   for (int s = 0; s < NS; ++s) dacc[s] = 0.0;
-  // features past D read feature D - 1 and rows past N row N - 1 (in bounds;
-  // they meet zeros of G^-1, q and u, or a weight of zero)
+  // features past D, all in the last tile, read feature D - 1 and rows past N row
+  // N - 1 (in bounds; they meet zeros of G^-1, q and u, or a weight of zero)
   // (byte offsets from a block's first row, as in gram_loop)
   uint32_t lastb[4];
 #pragma unroll
-  for (int s = 0; s < 4; ++s) lastb[s] = 8u * (uint32_t)min(16 * (NB - 1) + feat(s, g), D - 1);
+  for (int s = 0; s < 4; ++s) lastb[s] = last_tile_bytes(NB, quad_feature(s, g), D);
   const uint32_t rowb = 8u * (uint32_t)(m * D), gb = 16u * (uint32_t)g;
   auto fetch = [&](auto whole, double (&x)[NS], double& yv, int blk) {
     const int n0 = 16 * min(blk, nblk - 1);
     const char* const Xb = reinterpret_cast<const char*>(X + (size_t)n0 * D);
-    const uint32_t row = min(rowb, 8u * (uint32_t)(min(N - n0 - 1, 15) * D));
+    const uint32_t row = row_bytes(rowb, n0, N, D);
     const Pair* const xr = reinterpret_cast<const Pair*>(Xb + (row + gb));
 #pragma unroll
     for (int s = 0; s < NS - 4; s += 2) {
@@ -620,8 +605,8 @@ __device__ __forceinline__ void quad_pass_nb(Smem<C>& S, const double* X, const 
     double eta = 0.0, b = 0.0;
 #pragma unroll
     for (int s = 0; s < NS; ++s) {
-      eta = fma(x[s], S.q[feat(s, g)], eta);
-      if constexpr (RMHMC) b = fma(x[s], S.u[feat(s, g)], b);
+      eta = fma(x[s], S.q[quad_feature(s, g)], eta);
+      if constexpr (RMHMC) b = fma(x[s], S.u[quad_feature(s, g)], b);
     }
     eta = rows_sum(eta);
     if constexpr (RMHMC) b = rows_sum(b);
@@ -633,7 +618,7 @@ __device__ __forceinline__ void quad_pass_nb(Smem<C>& S, const double* X, const 
 #pragma unroll
       for (int s = 0; s < 4 * (tt + 1); ++s) {
         if (s == 4 * tt && tt > 0) v *= 2.0;
-        const double gi = REG ? T[REG ? i : 0] : S.Gi[feat(s, g) * C::LDX + 16 * tt + rf];
+        const double gi = REG ? T[REG ? i : 0] : S.Gi[quad_feature(s, g) * C::LDX + 16 * tt + rf];
         ++i;
         v = __builtin_amdgcn_mfma_f64_16x16x4f64(gi, x[s], v, 0, 0, 0);
       }
@@ -672,7 +657,7 @@ __device__ __forceinline__ void quad_pass_nb(Smem<C>& S, const double* X, const 
 #pragma unroll
   for (int s = 0; s < NS; ++s) {
     const double v = group_sum<16>(dacc[s]);
-    if (m == 0) S.part[w][feat(s, g)] = v;
+    if (m == 0) S.part[w][quad_feature(s, g)] = v;
   }
   __syncthreads();
   if (t < D) {
@@ -687,7 +672,7 @@ __device__ __forceinline__ void quad_pass_nb(Smem<C>& S, const double* X, const 
 template <class C>
 __device__ __forceinline__ void pass_quad(Smem<C>& S, const double* X, const double* y, int N, int D, double prior_var,
                                           bool rmhmc) {
-  by_width<C>(D, [&](auto nbc) __attribute__((always_inline)) {
+  by_width<C::MAXD>(D, [&](auto nbc) __attribute__((always_inline)) {
     constexpr int NB = decltype(nbc)::value;
     if (rmhmc)
       quad_pass_nb<C, NB, true>(S, X, y, N, D, prior_var);
