@@ -234,7 +234,7 @@ __global__ void __launch_bounds__(256) funnel_rmhmc_kernel(const FunnelArgs a) {
           const R na = R(1) + h * (cg + f.ce * ca), nb = h * (cd + f.ce * cb);
           const R ng = -h * (f.A * ca + f.B * cg), nd = R(1) - h * (f.A * cb + f.B * cd);
           const R da = na - ca, db = nb - cb, dg = ng - cg, dd = nd - cd;
-          R vn, pvn;
+          R vn, pvn, mx = R(0);
           bool go = false;
           if constexpr (kScreen) {
             vn = v0 + h * f.uv;
@@ -245,7 +245,6 @@ __global__ void __launch_bounds__(256) funnel_rmhmc_kernel(const FunnelArgs a) {
             const SpanDecision dec = bound(finite, mv, da, db, dg, dd, a.conv_tol, a.div_tol);
             go = more && dec == kGoOn;
             if (__any(active && (STEP ? !go : more && dec == kOpen))) {
-              R mx = R(0);
 #pragma unroll
               for (int k = 0; k < EPL; ++k)
                 mx = fmaxf(mx, fmaxf(fabsf(da * x0[k] + db * p0[k]), fabsf(dg * x0[k] + dd * p0[k])));
@@ -259,7 +258,6 @@ __global__ void __launch_bounds__(256) funnel_rmhmc_kernel(const FunnelArgs a) {
               go = more && isfinite(mx) && (double)mx < a.div_tol && (double)mx > a.conv_tol;
             }
           } else {
-            R mx = R(0);
 #pragma unroll
             for (int k = 0; k < EPL; ++k)
               mx = fmaxf(mx, fmaxf(fabsf(da * x0[k] + db * p0[k]), fabsf(dg * x0[k] + dd * p0[k])));
@@ -268,7 +266,6 @@ __global__ void __launch_bounds__(256) funnel_rmhmc_kernel(const FunnelArgs a) {
             pvn = pv0 - h * f.dHv;
             mx = nan_max(mx, nan_max(fabs(vn - vc), fabs(pvn - pvc)));
             if (!isfinite(na + nb + ng + nd)) mx = R(NAN);
-            if (active) norm = (double)mx;
           }
           if (active) {
             ca = na;
@@ -279,6 +276,7 @@ __global__ void __launch_bounds__(256) funnel_rmhmc_kernel(const FunnelArgs a) {
             pvc = pvn;
             sx = (ca * ca) * Sxx + (R(2) * ca * cb) * Sxp + (cb * cb) * Spp;
             xpx = (ca * cg) * Sxx + (ca * cd + cb * cg) * Sxp + (cb * cd) * Spp;
+            if constexpr (!kScreen) norm = (double)mx;
             ++n;
             ++n_fev;
           }
