@@ -23,27 +23,29 @@ namespace gjx {
 // After the two quad steps all lanes of a quad hold the quad total, so the
 // mirror steps pair whole quads / half rows, as an xor butterfly would.  Every
 // control used here reads a valid lane, so bound_ctrl (zero for lanes without a
-// source) never acts; with it set the move needs no initialised destination and
-// the compiler folds it into the float32 add or max that follows.
+// source) never acts.  FOLD sets it: the move then needs no initialised destination
+// and the compiler folds it into the float32 add or max that follows.  The sums are the
+// same; what changes is the order that the compiler finds for several sums one after
+// another, so kernels whose measurements say so turn it off.
 // ---------------------------------------------------------------------------
-template <int CTRL>
+template <int CTRL, bool FOLD = true>
 __device__ __forceinline__ float dpp_f32(float v) {
   return __builtin_bit_cast(
-      float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), CTRL, 0xF, 0xF, true));
+      float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), CTRL, 0xF, 0xF, FOLD));
 }
 
-template <int CTRL>
+template <int CTRL, bool FOLD = true>
 __device__ __forceinline__ double dpp_f64(double v) {
   uint64_t b = __builtin_bit_cast(uint64_t, v);
-  int lo = __builtin_amdgcn_update_dpp(0, (int)(uint32_t)b, CTRL, 0xF, 0xF, true);
-  int hi = __builtin_amdgcn_update_dpp(0, (int)(uint32_t)(b >> 32), CTRL, 0xF, 0xF, true);
+  int lo = __builtin_amdgcn_update_dpp(0, (int)(uint32_t)b, CTRL, 0xF, 0xF, FOLD);
+  int hi = __builtin_amdgcn_update_dpp(0, (int)(uint32_t)(b >> 32), CTRL, 0xF, 0xF, FOLD);
   return __builtin_bit_cast(double, ((uint64_t)(uint32_t)hi << 32) | (uint32_t)lo);
 }
 
-template <int CTRL>
-__device__ __forceinline__ float dpp(float v) { return dpp_f32<CTRL>(v); }
-template <int CTRL>
-__device__ __forceinline__ double dpp(double v) { return dpp_f64<CTRL>(v); }
+template <int CTRL, bool FOLD = true>
+__device__ __forceinline__ float dpp(float v) { return dpp_f32<CTRL, FOLD>(v); }
+template <int CTRL, bool FOLD = true>
+__device__ __forceinline__ double dpp(double v) { return dpp_f64<CTRL, FOLD>(v); }
 
 struct OpSum {
   template <class T> __device__ __forceinline__ static T f(T a, T b) { return a + b; }
@@ -53,19 +55,19 @@ struct OpMax {
 };
 
 // Reduce over an aligned group of W lanes (W power of two, 1..64).
-template <int W, class Op, class T>
+template <int W, class Op, bool FOLD = true, class T>
 __device__ __forceinline__ T group_reduce(T v) {
-  if constexpr (W >= 2) v = Op::f(v, dpp<0xB1>(v));
-  if constexpr (W >= 4) v = Op::f(v, dpp<0x4E>(v));
-  if constexpr (W >= 8) v = Op::f(v, dpp<0x141>(v));
-  if constexpr (W >= 16) v = Op::f(v, dpp<0x140>(v));
+  if constexpr (W >= 2) v = Op::f(v, dpp<0xB1, FOLD>(v));
+  if constexpr (W >= 4) v = Op::f(v, dpp<0x4E, FOLD>(v));
+  if constexpr (W >= 8) v = Op::f(v, dpp<0x141, FOLD>(v));
+  if constexpr (W >= 16) v = Op::f(v, dpp<0x140, FOLD>(v));
   if constexpr (W >= 32) v = Op::f(v, (T)__shfl_xor(v, 16, 64));
   if constexpr (W >= 64) v = Op::f(v, (T)__shfl_xor(v, 32, 64));
   return v;
 }
 
-template <int W, class T>
-__device__ __forceinline__ T group_sum(T v) { return group_reduce<W, OpSum>(v); }
+template <int W, bool FOLD = true, class T>
+__device__ __forceinline__ T group_sum(T v) { return group_reduce<W, OpSum, FOLD>(v); }
 template <int W, class T>
 __device__ __forceinline__ T group_max(T v) { return group_reduce<W, OpMax>(v); }
 

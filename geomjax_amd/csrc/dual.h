@@ -119,11 +119,11 @@ __device__ __forceinline__ float val(float x) { return x; }
 template <class T, int N> __device__ __forceinline__ T val(const Dual<T, N>& x) { return x.v; }
 
 // group reductions of dual numbers: component-wise sums
-template <int W, class T, int N>
+template <int W, bool FOLD = true, class T, int N>
 __device__ __forceinline__ Dual<T, N> group_sum(Dual<T, N> x) {
-  x.v = group_sum<W>(x.v);
+  x.v = group_sum<W, FOLD>(x.v);
 #pragma unroll
-  for (int i = 0; i < N; ++i) x.d[i] = group_sum<W>(x.d[i]);
+  for (int i = 0; i < N; ++i) x.d[i] = group_sum<W, FOLD>(x.d[i]);
   return x;
 }
 

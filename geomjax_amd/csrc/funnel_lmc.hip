@@ -49,6 +49,7 @@ __global__ void __launch_bounds__(256) funnel_lmc_kernel(const FunnelLmcArgs a) 
   const R halfDx = R(0.5 * Dx);
   const bool exact_sm = a.exact_sm != 0;
   const int T_steps = STEP ? 1 : a.T;
+  constexpr bool FOLD = folds_moves<R, LPC, EPL>();
 #define GJX_ON(k) (j0 + (k) < Dx)
 
   // diagonal inverse mass (the reference's inverse_mass_matrix, "fixed" power)
@@ -62,7 +63,7 @@ __global__ void __launch_bounds__(256) funnel_lmc_kernel(const FunnelLmcArgs a) 
 #pragma unroll
     for (int k = 0; k < EPL; ++k)
       if (GJX_ON(k)) s += log((double)mi[k]);
-    sum_log_mi = group_sum<LPC>(s) + log((double)miv);
+    sum_log_mi = group_sum<LPC, FOLD>(s) + log((double)miv);
   }
 
   // chain state: LMCState(position, logdensity, logdensity_grad, volume_adjustment)
@@ -81,7 +82,7 @@ __global__ void __launch_bounds__(256) funnel_lmc_kernel(const FunnelLmcArgs a) 
   for (int t = 0; t < T_steps; ++t) {
     // ---- position quantities at q0 (lmc.py:177-200) ----
     R loc_inc[EPL];
-    PosScalars<R> P = position_scalars<R, LPC, EPL>(x, v, mi, loc_inc, lg, a2, inv_s2, halfDx, miv);
+    PosScalars<R> P = position_scalars<R, LPC, EPL, FOLD>(x, v, mi, loc_inc, lg, a2, inv_s2, halfDx, miv);
 
     // ---- noise and velocity v0 = chol(M^-1 - alpha2 dl dl^T) z  (metrics.py:155-166) ----
     R z[EPL];
@@ -90,7 +91,7 @@ __global__ void __launch_bounds__(256) funnel_lmc_kernel(const FunnelLmcArgs a) 
     transition_noise<T, EPL>(a, c, t, j0, Dx, live, z, zv, uacc);
     R vx[EPL];
     R vv;
-    draw_velocity<R, LPC, EPL>(P, x, mi, loc_inc, z, zv, a2, alpha, miv, lg, j0, Dx, vx, vv);
+    draw_velocity<R, LPC, EPL, FOLD>(P, x, mi, loc_inc, z, zv, a2, alpha, miv, lg, j0, Dx, vx, vv);
     if (STEP && a.velocity != nullptr && live) {
 #pragma unroll
       for (int k = 0; k < EPL; ++k)
@@ -100,7 +101,7 @@ __global__ void __launch_bounds__(256) funnel_lmc_kernel(const FunnelLmcArgs a) 
 
     // ---- kinetic energy (metrics.py:168-186), float64 sums ----
     auto kinetic = [&](const PosScalars<R>& Q, const R (&xx)[EPL], const R (&vel)[EPL], R velv) -> double {
-      return lmc_kinetic<R, LPC, EPL>(Q, xx, vel, velv, mi, miv, j0, Dx, sum_log_mi, a.alpha2);
+      return lmc_kinetic<R, LPC, EPL, FOLD>(Q, xx, vel, velv, mi, miv, j0, Dx, sum_log_mi, a.alpha2);
     };
     const double K0 = kinetic(P, x, vx, vv);
 
@@ -117,7 +118,7 @@ __global__ void __launch_bounds__(256) funnel_lmc_kernel(const FunnelLmcArgs a) 
     for (int s = 0; s < a.L; ++s) {
       const bool on = s < Ls;
       if (!__any(on)) break;
-      if (on) lmc_step<R, LPC, EPL>(P, xc, vc, mi, vx, vv, dJ, eps, h, a2, inv_s2, halfDx, miv, exact_sm);
+      if (on) lmc_step<R, LPC, EPL, FOLD>(P, xc, vc, mi, vx, vv, dJ, eps, h, a2, inv_s2, halfDx, miv, exact_sm);
     }
 
     // ---- energy at the end (lmcmonge_energy, metrics.py:267-284) ----
@@ -127,7 +128,7 @@ __global__ void __launch_bounds__(256) funnel_lmc_kernel(const FunnelLmcArgs a) 
       double d1 = 0.0;
 #pragma unroll
       for (int k = 0; k < EPL; ++k) d1 += (double)xc[k] * (double)xc[k];
-      const double Sx = group_sum<LPC>(d1);
+      const double Sx = group_sum<LPC, FOLD>(d1);
       const double vd = (double)vc, s2 = a.sigma * a.sigma;
       logp1 = -0.5 * vd * vd / s2 - log(a.sigma) - 0.5 * kLog2Pi - 0.5 * exp(-vd) * Sx - 0.5 * (double)Dx * vd -
               0.5 * (double)Dx * kLog2Pi;
@@ -155,7 +156,7 @@ __global__ void __launch_bounds__(256) funnel_lmc_kernel(const FunnelLmcArgs a) 
       R xv = R(0);
 #pragma unroll
       for (int k = 0; k < EPL; ++k) xv += xc[k] * vx[k];
-      xv = group_sum<LPC>(xv);
+      xv = group_sum<LPC, FOLD>(xv);
       const R vg = -P.e * xv + vv * P.gv;
       const R mom_coef = a.exact_momentum ? a2 * vg : a2 * P.L * vg;  // metrics.py:243-255 (extra L)
       const R hv_v = (P.e * xv - (inv_s2 + R(0.5) * P.e * P.Sx) * vv) * P.isL;
@@ -240,7 +241,7 @@ __global__ void __launch_bounds__(256) funnel_lmc_kernel(const FunnelLmcArgs a) 
       R s1 = R(0);
 #pragma unroll
       for (int k = 0; k < EPL; ++k) s1 += x[k] * x[k];
-      const R sxf = group_sum<LPC>(s1);
+      const R sxf = group_sum<LPC, FOLD>(s1);
       const R e = exp(-v);
       const R gv = -v * inv_s2 - halfDx + R(0.5) * e * sxf;
       if (live) {

@@ -15,6 +15,19 @@
 namespace gjx {
 namespace lmc_ops {
 
+// Whether the group sums of a transition use folded moves (common.h, FOLD).  Not with 32
+// or 64 lanes of up to eight coordinates: the compiler then takes a half step's eight sums
+// one after another and waits for each exchange through LDS.  Nor in float32 where the moves
+// are few.  Time folded over not, 18 steps, four transitions, 9 | 1024 | 8192 chains (LPC x EPL):
+// float32 4x2 1.04 | 1.03 | 1.04, 8x2 1.02 | 1.01 | 1.00, 16x1 1.02 | 1.02 | 1.01, 16x4 0.99 | 0.99 | 0.99,
+// 16x8 0.99 | 0.99 | 1.00, 32x4 1.15 | 1.18 | 1.08, 64x2 1.25 | 1.24 | 1.07, 64x16 1.01 | 1.01 | 1.01;
+// float64 4x4 0.96 | 0.96 | 0.96, 16x4 0.91 | 0.91 | 0.92, 32x4 1.06 | 1.09 | 0.99, 32x8 1.03 | 1.05 | 1.08,
+// 32x16 0.94 | 0.95 | 1.00, 64x2 1.25 | 1.25 | 1.08, 64x16 0.95 | 0.95 | 0.97.
+template <class R, int LPC, int EPL>
+__device__ constexpr bool folds_moves() {
+  return sizeof(R) == sizeof(float) ? LPC == 16 && EPL >= 4 : LPC <= 16 || EPL > 8;
+}
+
 template <class R>
 struct PosScalars {
   R e, Sx, Smx, gv, L, sL, isL, dlv, Hdlv, igHdlv;
@@ -39,7 +52,7 @@ __device__ __forceinline__ PosScalars<R> pos_scalars(R v, R Sx, R Smx, R a2, R i
 
 // One half_step_omega (geomjax/lmcmonge/integrators.py:158-194) at the
 // position described by P, updating the velocity (vx, vv) and dJ.
-template <class R, int LPC, int EPL>
+template <class R, int LPC, int EPL, bool FOLD = true>
 __device__ __forceinline__ void half_step(const PosScalars<R>& P, const R (&x)[EPL], const R (&mi)[EPL], R (&vx)[EPL],
                                           R& vv, double& dJ, R a2, R inv_s2, R h, bool exact_sm) {
   R dl[EPL], dphig[EPL];
@@ -62,14 +75,14 @@ __device__ __forceinline__ void half_step(const PosScalars<R>& P, const R (&x)[E
     s6 += Hdl * dphig[k];
     s7 += Hdl * dl[k];
   }
-  s0 = group_sum<LPC>(s0);
-  s1 = group_sum<LPC>(s1);
-  s2 = group_sum<LPC>(s2);
-  s3 = group_sum<LPC>(s3);
-  s4 = group_sum<LPC>(s4);
-  s5 = group_sum<LPC>(s5);
-  s6 = group_sum<LPC>(s6);
-  s7 = group_sum<LPC>(s7);
+  s0 = group_sum<LPC, FOLD>(s0);
+  s1 = group_sum<LPC, FOLD>(s1);
+  s2 = group_sum<LPC, FOLD>(s2);
+  s3 = group_sum<LPC, FOLD>(s3);
+  s4 = group_sum<LPC, FOLD>(s4);
+  s5 = group_sum<LPC, FOLD>(s5);
+  s6 = group_sum<LPC, FOLD>(s6);
+  s7 = group_sum<LPC, FOLD>(s7);
   // log-scale coordinate contributions
   const R hv_v = (P.e * s2 - (inv_s2 + R(0.5) * P.e * P.Sx) * vv) * P.isL;
   const R gn_v = P.gv * P.isL;
@@ -100,7 +113,7 @@ __device__ __forceinline__ void half_step(const PosScalars<R>& P, const R (&x)[E
 
 // Scalars of the position (x, v) and the inclusive prefix of mi x^2 over the
 // chain's coordinates in lane order (the velocity draw's running sums).
-template <class R, int LPC, int EPL>
+template <class R, int LPC, int EPL, bool FOLD = true>
 __device__ __forceinline__ PosScalars<R> position_scalars(const R (&x)[EPL], R v, const R (&mi)[EPL], R (&loc_inc)[EPL],
                                                           int lg, R a2, R inv_s2, R halfDx, R miv) {
   R sx = R(0), smx = R(0);
@@ -113,8 +126,8 @@ __device__ __forceinline__ PosScalars<R> position_scalars(const R (&x)[EPL], R v
   const R off = group_exclusive_scan<LPC>(smx, lg);
 #pragma unroll
   for (int k = 0; k < EPL; ++k) loc_inc[k] += off;
-  sx = group_sum<LPC>(sx);
-  smx = group_sum<LPC>(smx);
+  sx = group_sum<LPC, FOLD>(sx);
+  smx = group_sum<LPC, FOLD>(smx);
   return pos_scalars<R>(v, sx, smx, a2, inv_s2, halfDx, miv);
 }
 
@@ -156,7 +169,7 @@ __device__ __forceinline__ void transition_noise(const FunnelLmcArgs& a, size_t 
 
 // Velocity v0 = chol(M^-1 - alpha2 dl dl^T) z (geomjax/lmcmonge/metrics.py:155-166)
 // with the exact lower factor of a diagonal-minus-rank-one matrix.
-template <class R, int LPC, int EPL>
+template <class R, int LPC, int EPL, bool FOLD = true>
 __device__ __forceinline__ void draw_velocity(const PosScalars<R>& P, const R (&x)[EPL], const R (&mi)[EPL],
                                               const R (&loc_inc)[EPL], const R (&z)[EPL], R zv, R a2, R alpha,
                                               R miv, int lg, int j0, int Dx, R (&vx)[EPL], R& vv) {
@@ -174,7 +187,7 @@ __device__ __forceinline__ void draw_velocity(const PosScalars<R>& P, const R (&
     acc2 += cj[k];
   }
   const R off2 = group_exclusive_scan<LPC>(acc2, lg);
-  const R tot2 = group_sum<LPC>(acc2);
+  const R tot2 = group_sum<LPC, FOLD>(acc2);
   R run = off2;
 #pragma unroll
   for (int k = 0; k < EPL; ++k) {
@@ -191,11 +204,11 @@ __device__ __forceinline__ void draw_velocity(const PosScalars<R>& P, const R (&
 
 // One lan_integrator step (geomjax/lmcmonge/integrators.py:52-156): half step of
 // the velocity, full step of the position, half step of the velocity.
-template <class R, int LPC, int EPL>
+template <class R, int LPC, int EPL, bool FOLD = true>
 __device__ __forceinline__ void lmc_step(PosScalars<R>& P, R (&xc)[EPL], R& vc, const R (&mi)[EPL], R (&vx)[EPL],
                                          R& vv, double& dJ, R eps, R h, R a2, R inv_s2, R halfDx, R miv,
                                          bool exact_sm) {
-  half_step<R, LPC, EPL>(P, xc, mi, vx, vv, dJ, a2, inv_s2, h, exact_sm);
+  half_step<R, LPC, EPL, FOLD>(P, xc, mi, vx, vv, dJ, a2, inv_s2, h, exact_sm);
   R sx = R(0), smx = R(0);
 #pragma unroll
   for (int k = 0; k < EPL; ++k) {
@@ -204,17 +217,17 @@ __device__ __forceinline__ void lmc_step(PosScalars<R>& P, R (&xc)[EPL], R& vc, 
     smx += mi[k] * xc[k] * xc[k];
   }
   vc = vc + eps * vv;
-  sx = group_sum<LPC>(sx);
-  smx = group_sum<LPC>(smx);
+  sx = group_sum<LPC, FOLD>(sx);
+  smx = group_sum<LPC, FOLD>(smx);
   P = pos_scalars<R>(vc, sx, smx, a2, inv_s2, halfDx, miv);
-  half_step<R, LPC, EPL>(P, xc, mi, vx, vv, dJ, a2, inv_s2, h, exact_sm);
+  half_step<R, LPC, EPL, FOLD>(P, xc, mi, vx, vv, dJ, a2, inv_s2, h, exact_sm);
 }
 
 
 // Kinetic energy of the lmcmonge metric (geomjax/lmcmonge/metrics.py:168-186) in
 // float64 sums: -(log L - sum log mi)/2 + |v|_M^2 / 2 + alpha2 (v . g)^2 / 2,
 // g = (-e x, gv) the full gradient.
-template <class R, int LPC, int EPL>
+template <class R, int LPC, int EPL, bool FOLD = true>
 __device__ __forceinline__ double lmc_kinetic(const PosScalars<R>& Q, const R (&xx)[EPL], const R (&vel)[EPL], R velv,
                                               const R (&mi)[EPL], R miv, int j0, int Dx, double sum_log_mi,
                                               double alpha2) {
@@ -224,8 +237,8 @@ __device__ __forceinline__ double lmc_kinetic(const PosScalars<R>& Q, const R (&
     if (j0 + k < Dx) svm += (double)val(vel[k]) * (double)val(vel[k]) / (double)val(mi[k]);
     xv += (double)val(xx[k]) * (double)val(vel[k]);
   }
-  svm = group_sum<LPC>(svm) + (double)val(velv) * (double)val(velv) / (double)val(miv);
-  xv = group_sum<LPC>(xv);
+  svm = group_sum<LPC, FOLD>(svm) + (double)val(velv) * (double)val(velv) / (double)val(miv);
+  xv = group_sum<LPC, FOLD>(xv);
   const double vg = -(double)val(Q.e) * xv + (double)val(velv) * (double)val(Q.gv);  // v . g
   return -0.5 * (log((double)val(Q.L)) - sum_log_mi) + 0.5 * svm + 0.5 * alpha2 * vg * vg;
 }

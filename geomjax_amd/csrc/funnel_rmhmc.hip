@@ -45,6 +45,11 @@ __global__ void __launch_bounds__(256) funnel_rmhmc_kernel(const FunnelArgs a) {
   // float32 (the tuned form) iterates in span{x0, p0}; float64 updates every
   // coordinate, the reference's own operation order
   constexpr bool kSpan = sizeof(T) == sizeof(float);
+  // folded moves (common.h) but where the float32 sums take exchanges through LDS: time
+  // folded over not, 18 steps, four transitions, 9 | 1024 | 8192 chains (LPC x EPL): 32x1 1.03 | 1.03 | 1.03,
+  // 32x4 1.04 | 1.03 | 1.00, 32x8 0.99 | 0.98 | 1.00, 64x2 1.02 | 1.02 | 1.01, 64x8 1.02 | 1.02 | 1.02; with
+  // fewer lanes 0.98..1.02, in float64 0.94..0.98.
+  constexpr bool FOLD = sizeof(R) == 8 || LPC < 32 || (LPC == 32 && EPL >= 8);
   const int tid = blockIdx.x * 256 + threadIdx.x;
   const int chain = tid / LPC;
   const int lg = tid % LPC;
@@ -118,7 +123,7 @@ __global__ void __launch_bounds__(256) funnel_rmhmc_kernel(const FunnelArgs a) {
         acc += x[k] * x[k];
         loc_inc[k] = acc;
       }
-      sx = group_sum<LPC>(acc);
+      sx = group_sum<LPC, FOLD>(acc);
       const R off1 = group_exclusive_scan<LPC>(acc, lg);
       const R e = exp(-v);
       const R a2e2 = a2 * e * e;
@@ -136,7 +141,7 @@ __global__ void __launch_bounds__(256) funnel_rmhmc_kernel(const FunnelArgs a) {
         acc2 += cj[k];
       }
       const R off2 = group_exclusive_scan<LPC>(acc2, lg);
-      const R tot2 = group_sum<LPC>(acc2);
+      const R tot2 = group_sum<LPC, FOLD>(acc2);
       R run = off2;
 #pragma unroll
       for (int k = 0; k < EPL; ++k) {
@@ -166,8 +171,8 @@ __global__ void __launch_bounds__(256) funnel_rmhmc_kernel(const FunnelArgs a) {
         a1 += x[k] * px[k];
         a3 += (double)px[k] * (double)px[k];
       }
-      xpx = group_sum<LPC>(a1);
-      const double pp = group_sum<LPC>(a3) + (double)pv * pv;
+      xpx = group_sum<LPC, FOLD>(a1);
+      const double pp = group_sum<LPC, FOLD>(a3) + (double)pv * pv;
       const double e = exp(-(double)v);
       const double gv = -(double)v / (a.sigma * a.sigma) - 0.5 * Dx + 0.5 * e * (double)sx;
       const double gp = -e * (double)xpx + gv * (double)pv;
@@ -180,7 +185,7 @@ __global__ void __launch_bounds__(256) funnel_rmhmc_kernel(const FunnelArgs a) {
         a4 += r * r;
       }
       const double rv = (double)pv - cp * gv;
-      const double perp2 = group_sum<LPC>(a4) + rv * rv;
+      const double perp2 = group_sum<LPC, FOLD>(a4) + rv * rv;
       const double Tk = 0.5 * monge_quad(pp, perp2, gg, a.alpha2) + 0.5 * log(1.0 + a.alpha2 * gg) +
                         0.5 * (double)D * kLog2Pi;
       H0 = -logp + Tk;
@@ -224,7 +229,7 @@ __global__ void __launch_bounds__(256) funnel_rmhmc_kernel(const FunnelArgs a) {
         R spp = R(0);
 #pragma unroll
         for (int k = 0; k < EPL; ++k) spp += p0[k] * p0[k];
-        const R Sxx = sx, Sxp = xpx, Spp = group_sum<LPC>(spp);
+        const R Sxx = sx, Sxp = xpx, Spp = group_sum<LPC, FOLD>(spp);
         constexpr bool kScreen = span_screens<LPC, EPL>();
         const SpanBound bound((float)Sxx, (float)Spp);
         R ca = R(1), cb = R(0), cg = R(0), cd = R(1);
@@ -248,7 +253,7 @@ __global__ void __launch_bounds__(256) funnel_rmhmc_kernel(const FunnelArgs a) {
 #pragma unroll
               for (int k = 0; k < EPL; ++k)
                 mx = fmaxf(mx, fmaxf(fabsf(da * x0[k] + db * p0[k]), fabsf(dg * x0[k] + dd * p0[k])));
-              mx = group_reduce<LPC, OpMax>(mx);
+              mx = group_reduce<LPC, OpMax, FOLD>(mx);
               mx = nan_max(mx, mv);
               // the per-coordinate max drops NaN; a non-finite coefficient (or step
               // start sum, through the field) makes the norm NaN instead
@@ -261,7 +266,7 @@ __global__ void __launch_bounds__(256) funnel_rmhmc_kernel(const FunnelArgs a) {
 #pragma unroll
             for (int k = 0; k < EPL; ++k)
               mx = fmaxf(mx, fmaxf(fabsf(da * x0[k] + db * p0[k]), fabsf(dg * x0[k] + dd * p0[k])));
-            mx = group_reduce<LPC, OpMax>(mx);
+            mx = group_reduce<LPC, OpMax, FOLD>(mx);
             vn = v0 + h * f.uv;
             pvn = pv0 - h * f.dHv;
             mx = nan_max(mx, nan_max(fabs(vn - vc), fabs(pvn - pvc)));
@@ -306,10 +311,10 @@ __global__ void __launch_bounds__(256) funnel_rmhmc_kernel(const FunnelArgs a) {
         }
         const R vn = v0 + h * f.uv;
         const R pvn = pv0 - h * f.dHv;
-        mx = group_reduce<LPC, NanMax>(mx);
+        mx = group_reduce<LPC, NanMax, FOLD>(mx);
         mx = nan_max(mx, nan_max(fabs(vn - vc), fabs(pvn - pvc)));
-        s1 = group_sum<LPC>(s1);
-        s2 = group_sum<LPC>(s2);
+        s1 = group_sum<LPC, FOLD>(s1);
+        s2 = group_sum<LPC, FOLD>(s2);
         if (active) {
           vc = vn;
           pvc = pvn;
@@ -345,8 +350,8 @@ __global__ void __launch_bounds__(256) funnel_rmhmc_kernel(const FunnelArgs a) {
         }
         vc = on ? vc + h * f.uv : vc;
         pvc = on ? pvc - h * f.dHv : pvc;
-        sx = group_sum<LPC>(s1);
-        xpx = group_sum<LPC>(s2);
+        sx = group_sum<LPC, FOLD>(s1);
+        xpx = group_sum<LPC, FOLD>(s2);
         n_fev += on ? 1 : 0;
       }
     }
@@ -363,9 +368,9 @@ __global__ void __launch_bounds__(256) funnel_rmhmc_kernel(const FunnelArgs a) {
         d2 += (double)xc[k] * (double)pc[k];
         d3 += (double)pc[k] * (double)pc[k];
       }
-      const double Sx = group_sum<LPC>(d1);
-      const double Xp = group_sum<LPC>(d2);
-      const double pp = group_sum<LPC>(d3) + (double)pvc * pvc;
+      const double Sx = group_sum<LPC, FOLD>(d1);
+      const double Xp = group_sum<LPC, FOLD>(d2);
+      const double pp = group_sum<LPC, FOLD>(d3) + (double)pvc * pvc;
       const double vd = (double)vc;
       const double s2 = a.sigma * a.sigma;
       const double e = exp(-vd);
@@ -381,7 +386,7 @@ __global__ void __launch_bounds__(256) funnel_rmhmc_kernel(const FunnelArgs a) {
         d4 += r * r;
       }
       const double rv = (double)pvc - cp * gv;
-      const double perp2 = group_sum<LPC>(d4) + rv * rv;
+      const double perp2 = group_sum<LPC, FOLD>(d4) + rv * rv;
       // funnel log density (examples/funnel/main.py:34-39)
       logp1 = -0.5 * vd * vd / s2 - log(a.sigma) - 0.5 * kLog2Pi - 0.5 * e * Sx - 0.5 * (double)Dx * vd -
               0.5 * (double)Dx * kLog2Pi;
@@ -476,7 +481,7 @@ __global__ void __launch_bounds__(256) funnel_rmhmc_kernel(const FunnelArgs a) {
       R s1 = R(0);
 #pragma unroll
       for (int k = 0; k < EPL; ++k) s1 += x[k] * x[k];
-      const R sxf = group_sum<LPC>(s1);
+      const R sxf = group_sum<LPC, FOLD>(s1);
       const R e = exp(-v);
       const R gv = -v * inv_s2 - halfDx + R(0.5) * e * sxf;
       if (live) {
