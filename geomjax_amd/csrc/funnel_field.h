@@ -47,8 +47,12 @@ __device__ __forceinline__ FieldCoef<R> field_coef(R v, R pv, R sx, R xpx, R a2,
 //   norm >= mv  and  norm <= max(|da| X + |db| P, |dg| X + |dd| P, mv),
 // so mv > tol with the upper bound below the divergence limit goes on, an upper
 // bound within tol has converged, and a non-finite change (norm NaN) stops.
-// Everything else is kOpen: the norm itself has to be formed.  Comparisons with
-// NaN are false, which leads there.
+// Everything else is kOpen: the norm itself has to be formed.
+// A term of the upper bound is NaN only as 0 times an infinite X or P, and fmaxf drops
+// it.  An infinite |x0|^2 makes the field's coefficients NaN (finite is false); with
+// an infinite |p0|^2 and a step other than 0 the change's coefficient of p0 in x is not 0 in
+// the first iterate, so the other term is infinite (kOpen), and the next iterate's field
+// is NaN.  With a step of 0 all four coefficients are 0 and the norm is mv.
 enum SpanDecision { kStop, kGoOn, kOpen };
 
 struct SpanBound {
