@@ -325,9 +325,10 @@ hipError_t launch_diagnostics(const void* x, int dtype, int N, int C, int D, int
       const size_t lds = (size_t)(N + diag::kPad) * diag::kRow * sizeof(double);
       const bool lags = ess != nullptr;
       auto k = lane_d ? diag::lag_block_kernel<T, true> : diag::lag_block_kernel<T, false>;
-      // few coordinates: 64 chains a round, as many workgroups as the partial sums have room for
-      // (without lag sums there are none: a few chains each)
-      const int per = !lags && lane_d ? std::max(1, C / 1024) : lane_d ? tc : (ntiles * 64 >= C ? 64 : (C + ntiles - 1) / ntiles);
+      // chains per workgroup: a tile as the partial sums are laid out (without lag sums there
+      // are none: a few), or one for each lane (fewer workgroups than tiles)
+      static_assert(diag::kMaxTile <= 64, "64 chains a workgroup need no more partial sums than tiles");
+      const int per = !lane_d ? 64 : lags ? tc : std::max(1, C / 1024);
       ntiles = (C + per - 1) / per;
       hipError_t e = hipFuncSetAttribute((const void*)k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
       if (e != hipSuccess) return e;
