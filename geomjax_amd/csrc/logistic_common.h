@@ -348,6 +348,11 @@ __device__ __forceinline__ void gram_pass_nb(Smem<C>& S, const double* X, const 
   if constexpr (C::H == 1) {
     if (w == 0) {
       add(S.tile);
+      // G takes the space of the tiles: every lane's reads before any lane's stores
+      // (the LDS accesses of one wave complete in order; this keeps the compiler to it)
+      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
       store(std::integral_constant<int, 0>{});
     }
   } else {
