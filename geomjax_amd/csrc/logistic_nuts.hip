@@ -24,6 +24,15 @@
 // next step from that end.  The tree building (lnuts_tree) is written once over
 // a load(end) / step(h) pair.  U-turn checkpoints ([NA][M][64] doubles) follow
 // the Smem block in dynamic LDS.
+//
+// The tree is inlined into the kernels by force: as a function of its own (the compiler's
+// choice once the passes had grown) it took the chain's state through scratch memory.  Two
+// workgroups share a CU: registers are bounded to 256 a lane, 139 and 187 of them
+// spilled outside the passes' loops.  Transitions of up to four leaves | up to sixteen,
+// RMHMC, a call of that function at one workgroup per CU -> now: 2048 x 64 with 256 chains
+// 6.24 | 29.3 -> 2.72 | 12.5 ms, with 600 chains 18.5 -> 6.8 ms, 100 x 16 with 2048 chains
+// 8.8 | 40.4 -> 1.10 | 4.84 ms, 20 x 2 with one chain 0.281 | 0.278 -> 0.112 | 0.110 ms (inlined with one
+// workgroup per CU 0.105 | 0.102, but 1.77 | 7.85 at 100 x 16).
 #include "common.h"
 #include "logistic.h"
 #include "logistic_common.h"
@@ -66,7 +75,7 @@ struct Uniform {
   int c;
   uint64_t tt;
   uint32_t k0, k1;
-  __device__ double operator()(const double* host, size_t idx, uint32_t stream, uint32_t i) const {
+  __device__ __forceinline__ double operator()(const double* host, size_t idx, uint32_t stream, uint32_t i) const {
     if (host != nullptr) return host[idx];
     u32x4 r = philox4x32_10(u32x4{(uint32_t)c, (uint32_t)tt, stream + i, (uint32_t)(tt >> 32)}, k0, k1);
     return u01_f64(r.x, r.y) - 0.5 * (1.0 / 9007199254740992.0);
@@ -81,7 +90,7 @@ struct Uniform {
 // and returns its energy.  Every decision is taken on block-reduced values, the
 // same in all lanes, so the workgroup stays uniform.
 template <class Load, class Step>
-__device__ TreeOut lnuts_tree(const Pt& s0, double H0, Load load, Step step, const Uniform& uniform,
+__device__ __forceinline__ TreeOut lnuts_tree(const Pt& s0, double H0, Load load, Step step, const Uniform& uniform,
                               const NutsArgs& nu, double eps, double div_threshold, Smem<C>& S, double* ck, int c,
                               Pt& left, Pt& right, Prop& prop) {
   const int t = threadIdx.x;
@@ -244,7 +253,7 @@ __device__ __forceinline__ void load_state_and_noise(const LogisticArgs& a, Smem
 
 // The proposal's state (gradient g given per lane), the trajectory's ends, row
 // tails past D and NUTSInfo.
-__device__ void write_outputs(const LogisticArgs& a, const NutsArgs& nu, int c, int D, const Prop& prop, double g,
+__device__ __forceinline__ void write_outputs(const LogisticArgs& a, const NutsArgs& nu, int c, int D, const Prop& prop, double g,
                               const Pt& left, const Pt& right, const TreeOut& t_out) {
   const int t = threadIdx.x, Dp = a.Dmax;
   const size_t row = (size_t)c * Dp;
@@ -280,7 +289,7 @@ using namespace lnuts;
 // ---------------------------------------------------------------------------
 // NUTS with the RMHMC implicit midpoint (geomjax/rmhmc/nuts.py)
 // ---------------------------------------------------------------------------
-__global__ void __launch_bounds__(NT, 1) logistic_nuts_f64_kernel(const LogisticArgs a, const NutsArgs nu) {
+__global__ void __launch_bounds__(NT, 2) logistic_nuts_f64_kernel(const LogisticArgs a, const NutsArgs nu) {
   extern __shared__ __align__(16) unsigned char smem_raw[];
   Smem<C>& S = *reinterpret_cast<Smem<C>*>(smem_raw);
   double* const ck = reinterpret_cast<double*>(smem_raw + sizeof(Smem<C>));
@@ -403,7 +412,7 @@ __global__ void __launch_bounds__(NT, 1) logistic_nuts_f64_kernel(const Logistic
 // ---------------------------------------------------------------------------
 // NUTS with the general-metric LMC integrator (geomjax/lmcmc/nuts.py)
 // ---------------------------------------------------------------------------
-__global__ void __launch_bounds__(NT, 1) logistic_nuts_lmc_f64_kernel(const LogisticArgs a, const NutsArgs nu) {
+__global__ void __launch_bounds__(NT, 2) logistic_nuts_lmc_f64_kernel(const LogisticArgs a, const NutsArgs nu) {
   extern __shared__ __align__(16) unsigned char smem_raw[];
   Smem<C>& S = *reinterpret_cast<Smem<C>*>(smem_raw);
   double* const ck = reinterpret_cast<double*>(smem_raw + sizeof(Smem<C>));
