@@ -59,7 +59,7 @@ struct Smem {
 };
 
 __device__ __forceinline__ double block_sum(Smem& S, double v) {
-  v = group_sum<64>(v);
+  v = group_sum<64, false>(v);
   __syncthreads();
   if (threadIdx.x % 64 == 0) S.red[threadIdx.x / 64] = v;
   __syncthreads();
@@ -67,7 +67,7 @@ __device__ __forceinline__ double block_sum(Smem& S, double v) {
 }
 
 __device__ __forceinline__ double block_max(Smem& S, double v) {
-  v = group_reduce<64, NanMax>(v);
+  v = group_reduce<64, NanMax, false>(v);
   __syncthreads();
   if (threadIdx.x % 64 == 0) S.red[threadIdx.x / 64] = v;
   __syncthreads();
